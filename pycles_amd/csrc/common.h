@@ -160,6 +160,14 @@ __device__ __forceinline__ uint3 xcd_tile() {
     return make_uint3(idx % gx, xcd * band + t % band, t / band);
 }
 
+// The same for a linear list of n work items, one per block of a 1-D grid of
+// n blocks: XCD x works on a contiguous share of the list (n / 8 items, one
+// more for the first n % 8 XCDs).  A bijection of [0, n).
+__device__ __forceinline__ long long xcd_band(long long b, long long n) {
+    const long long q = n / 8, r = n % 8, x = b % 8;
+    return x * q + (x < r ? x : r) + b / 8;
+}
+
 // ---------------------------------------------------------------------------
 // Interpolants.  The expression trees follow reference
 // Csrc/advection_interpolation.h (interp_4 :12-14, interp_6 :20-24,
