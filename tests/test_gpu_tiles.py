@@ -48,3 +48,75 @@ def test_layout_tiles(n, gw, precision):
     # without a base: the values themselves
     _capi.layout_egress(_dims(n, gw), dev.data_ptr(), back.data_ptr(), None, code, D.stream())
     assert np.array_equal(back.cpu().numpy(), want.astype(np.float64)[:, j][:, :, i].transpose(2, 1, 0))
+
+
+@pytest.mark.parametrize("n,gw", [((70, 9, 13), 3), ((6, 6, 5), 3), ((65, 8, 40), 2)])
+def test_sgs_and_diffusion_tiles_bitwise(n, gw):
+    """The SGS and diffusion marches over partial column tiles and uneven z
+    chunks, FP64, bitwise against the oracle (each operator's calls apart as
+    well as in one pass)."""
+    import torch
+    from oracle import oracle as O
+    from pycles_amd import _capi
+    from pycles_amd import _device as D
+    nx, ny, nz = n
+    nzg = nz + 2 * gw
+    rng = np.random.default_rng(nx)
+    dx = (50.0, 60.0, 20.0)
+    dims, odims = _dims(n, gw, dx), O.make_dims(nx, ny, nz, gw, *dx)
+    alpha = 0.8 + 0.01 * np.arange(nzg)
+    half = alpha - 0.004
+    prof = {"rho0": 1.0 / alpha, "rho0_half": 1.0 / half, "alpha0": alpha, "alpha0_half": half,
+            "p0": 1e5 - 200.0 * np.arange(nzg), "p0_half": 1e5 - 200.0 * np.arange(nzg) + 90.0}
+    oref = O.Ref(prof["p0"], prof["p0_half"], alpha, half, prof["rho0"], prof["rho0_half"])
+    dp = {k: _dev(v) for k, v in prof.items()}
+    ref = _capi.Ref(*[dp[k].data_ptr() for k in ("rho0", "rho0_half", "alpha0", "alpha0_half", "p0", "p0_half")])
+    f = {k: rng.standard_normal((nzg, ny, nx)) for k in ("u", "v", "w", "s", "qt", "n2", "tu", "tv", "tw", "ts", "tq")}
+    f["T"] = 290.0 + rng.standard_normal((nzg, ny, nx))
+    f["n2"] *= 1e-3
+
+    def ghosted(a):
+        return np.ascontiguousarray(np.pad(a.transpose(2, 1, 0), ((gw, gw), (gw, gw), (0, 0)), mode="wrap"))
+
+    sim = O.OracleSimulation(odims, oref, True, O.Lookup(np.linspace(100.0, 380.0, 16), np.linspace(1.0, 2.0, 16)),
+                             sgs={"cs": 0.17, "prt": 1.0 / 3.0})
+    for k in ("u", "v", "w", "s", "qt"):
+        sim.pv(k)[...] = ghosted(f[k])
+        sim.pt(k)[...] = ghosted(f["t" + k[0]])
+    sim.dv["buoyancy_frequency"][...] = ghosted(f["n2"])
+    sim.dv["temperature"][...] = ghosted(f["T"])
+    sim.kinematics_update()
+    sim.sgs_update()
+    t = {k: _dev(v) for k, v in f.items()}
+    smag, nu, dif = (torch.full((nzg, ny, nx), -1.0, dtype=torch.float64, device="cuda") for _ in range(3))
+    vel = [t[k].data_ptr() for k in ("u", "v", "w")]
+    st = D.stream()
+    _capi.sgs_smagorinsky(dims, vel, t["n2"].data_ptr(), 0.17, 1.0 / 3.0, smag.data_ptr(), nu.data_ptr(), dif.data_ptr(),
+                          D.F64, st)
+    lv = slice(1, nzg - 1)
+
+    def inner(a):
+        return np.asarray(a)[gw:-gw, gw:-gw].transpose(2, 1, 0)
+
+    assert np.array_equal(smag.cpu().numpy()[lv], inner(sim.smag)[lv])
+    assert np.array_equal(nu.cpu().numpy()[lv], inner(sim.dv["viscosity"])[lv])
+    assert np.array_equal(dif.cpu().numpy()[lv], inner(sim.dv["diffusivity"])[lv])
+    # the ghost levels' outer ends, which the reference leaves at zero
+    for a in (smag, nu, dif):
+        assert not a[0].any() and not a[-1].any()
+    # their periodic images (the oracle's own stop at ghost column 1, where
+    # the reference reads before its array)
+    sim.smag[...] = ghosted(smag.cpu().numpy())
+    sim.dv["viscosity"][...] = ghosted(nu.cpu().numpy())
+    sim.dv["diffusivity"][...] = ghosted(dif.cpu().numpy())
+    sim.scalar_diffusion_update()
+    sim.momentum_diffusion_update()
+    S, M, E = _capi.DIFF_SCALARS, _capi.DIFF_MOMENTUM, _capi.DIFF_ENTROPY_SOURCE
+    for flags in ([S | M | E], [S, M | E], [S, M, E]):
+        tend = {k: _dev(f["t" + k]) for k in "uvwsq"}
+        for fl in flags:
+            _capi.diffusion(dims, ref, vel, [tend[k].data_ptr() for k in "uvw"] if fl & M else None,
+                            [t["s"].data_ptr(), t["qt"].data_ptr()], [tend["s"].data_ptr(), tend["q"].data_ptr()], None,
+                            nu.data_ptr(), dif.data_ptr(), smag.data_ptr(), t["T"].data_ptr(), fl, D.F64, st)
+        for k, n_ in (("u", "u"), ("v", "v"), ("w", "w"), ("s", "s"), ("q", "qt")):
+            assert np.array_equal(tend[k].cpu().numpy()[gw:-gw], inner(sim.pt(n_))[gw:-gw]), (flags, n_)
