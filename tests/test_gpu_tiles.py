@@ -120,3 +120,64 @@ def test_sgs_and_diffusion_tiles_bitwise(n, gw):
                             nu.data_ptr(), dif.data_ptr(), smag.data_ptr(), t["T"].data_ptr(), fl, D.F64, st)
         for k, n_ in (("u", "u"), ("v", "v"), ("w", "w"), ("s", "s"), ("q", "qt")):
             assert np.array_equal(tend[k].cpu().numpy()[gw:-gw], inner(sim.pt(n_))[gw:-gw]), (flags, n_)
+
+
+@pytest.mark.parametrize("n,gw", [((8, 6, 3), 3), ((9, 7, 5), 5), ((64, 33, 20), 3), ((13, 1, 11), 2), ((1, 3, 4), 4)])
+@pytest.mark.parametrize("precision,shift", [("f64", 0), ("f32", 0), ("f32", 1), ("f64", 1)])
+def test_rk3_stage_tiles(n, gw, precision, shift):
+    """The RK3 stage over planes that do and do not divide into 16-byte
+    accesses, fields off a 16-byte boundary (shift), columns no deeper than
+    their ghost rim, and every boundary type, bitwise against numpy in the
+    field's precision (the update uses uncontracted + and *)."""
+    import torch
+    from pycles_amd import _capi
+    from pycles_amd import _device as D
+    nx, ny, nz = n
+    nzg, N = nz + 2 * gw, nx * ny * (nz + 2 * gw)
+    np_t = np.float64 if precision == "f64" else np.float32
+    code = D.precision_code(precision)
+    bcs = [1.0, -1.0, 2.0, -0.5]
+    rng = np.random.default_rng(7)
+    val, ten, cpy = (rng.standard_normal((4, nzg, ny, nx)).astype(np_t) for _ in range(3))
+    sl = slice(gw, gw + nz)
+    dt = 0.7
+
+    def up(a):
+        buf = torch.zeros(4 * N + 4, dtype=D.torch_dtype(code), device="cuda")
+        buf[shift:shift + 4 * N] = _dev(a).reshape(-1)
+        return buf, [buf.data_ptr() + (shift + q * N) * buf.element_size() for q in range(4)]
+
+    def down(b):
+        return b[shift:shift + 4 * N].cpu().numpy().reshape(4, nzg, ny, nx)
+
+    for rk in range(3):
+        for zero in (0, 1):
+            bv, pv = up(val)
+            bt, pt = up(ten)
+            bc_, pc = up(cpy)
+            _capi.rk3_stage(_dims(n, gw), pv, pt, pc, bcs, rk, dt, code, D.stream(), zero)
+            d = np_t(dt)
+            x = val + ten * d
+            want_c = cpy.copy()
+            if rk == 0:
+                want_c[:, sl] = val[:, sl]
+            elif rk == 1:
+                x = np_t(0.75) * cpy + np_t(0.25) * x
+            else:
+                x = np_t(1.0 / 3.0) * cpy + np_t(2.0 / 3.0) * x
+            want = val.copy()
+            want[:, sl] = x[:, sl]
+            for q, bc in enumerate(bcs):
+                f = want[q]
+                for m in range(gw):
+                    if bc == 1.0:
+                        f[gw - 1 - m], f[nzg - gw + m] = f[gw + m], f[nzg - gw - 1 - m]
+                    elif bc == 2.0:
+                        f[gw - 1 - m], f[nzg - gw + m] = f[gw], f[nzg - gw - 1]
+                    elif m == 0:
+                        f[gw - 1] = f[nzg - gw] = 0.0
+                    else:
+                        f[gw - 1 - m], f[nzg - gw + m] = np_t(bc) * f[gw - 1 + m], np_t(bc) * f[nzg - gw - m]
+            assert np.array_equal(down(bv), want), (rk, zero)
+            assert np.array_equal(down(bc_), want_c), (rk, zero)
+            assert np.array_equal(down(bt), np.zeros_like(ten) if zero else ten), (rk, zero)
