@@ -181,3 +181,68 @@ def test_rk3_stage_tiles(n, gw, precision, shift):
             assert np.array_equal(down(bv), want), (rk, zero)
             assert np.array_equal(down(bc_), want_c), (rk, zero)
             assert np.array_equal(down(bt), np.zeros_like(ten) if zero else ten), (rk, zero)
+
+
+@pytest.mark.parametrize("n,gw", [((8, 8, 6), 3), ((9, 7, 5), 5), ((68, 61, 4), 2), ((1, 1, 2), 2), ((256, 130, 13), 3)])
+@pytest.mark.parametrize("precision", ["f64", "f32"])
+def test_statistics_tiles(n, gw, precision):
+    """Level statistics over planes that do and do not divide into 16-byte
+    accesses and shares, with and without a second factor and a mask, and the
+    cloud statistics over partial column groups and depths that do not divide
+    by the wavefronts, against numpy.  Sums of N terms in two orders differ by
+    at most N eps times the sum of their magnitudes; extremes and counts are
+    exact."""
+    import torch
+    from pycles_amd import _capi
+    from pycles_amd import _device as D
+    nx, ny, nz = n
+    nzg, N = nz + 2 * gw, nx * ny
+    code = D.precision_code(precision)
+    np_t = np.float64 if precision == "f64" else np.float32
+    rng = np.random.default_rng(11)
+    a, b = (rng.standard_normal((nzg, ny, nx)).astype(np_t) for _ in range(2))
+    mask = (rng.random((nzg, ny, nx)) < 0.3).astype(np_t)
+    mask[0] = 0.0
+    ba, bb = 5.0 + rng.random(nzg), -2.0 + rng.random(nzg)
+    dims = _dims(n, gw)
+    ws = torch.empty(_capi.horizontal_stats_workspace_bytes(dims), dtype=torch.uint8, device="cuda")
+    ta, tb, tm, tba, tbb = (_dev(x) for x in (a, b, mask, ba, bb))
+    eps = np.finfo(np.float64).eps
+    for second in (False, True):
+        for masked in (False, True):
+            out = torch.empty((6, nzg), dtype=torch.float64, device="cuda")
+            _capi.horizontal_stats(dims, ta.data_ptr(), tba.data_ptr(), tb.data_ptr() if second else None,
+                                   tbb.data_ptr() if second else None, tm.data_ptr() if masked else None, code,
+                                   out.data_ptr(), ws.data_ptr(), D.stream())
+            got = out.cpu().numpy()
+            v = a.astype(np.float64) + ba[:, None, None]
+            if second:
+                v = v * (b.astype(np.float64) + bb[:, None, None])
+            m = mask.astype(np.float64) if masked else np.ones_like(v)
+            cnt = m.sum(axis=(1, 2))
+            div = np.maximum(cnt, 1.0) if masked else float(N)
+            for q in range(3):
+                want = (v ** (q + 1) * m).sum(axis=(1, 2)) / div
+                mag = (np.abs(v) ** (q + 1) * m).sum(axis=(1, 2)) / div
+                assert np.all(np.abs(got[q] - want) <= (N + 8) * eps * mag), (second, masked, q)
+            w = np.where(m != 0.0, v, np.nan)
+            for k in range(nzg):
+                hi, lo = (-9e12, 9e12) if not m[k].any() else (np.nanmax(w[k]), np.nanmin(w[k]))
+                assert got[3, k] == hi and got[4, k] == lo
+            assert np.array_equal(got[5], cnt)
+    ql = np.where(rng.random((nzg, ny, nx)) < 0.2, rng.random((nzg, ny, nx)), 0.0).astype(np_t)
+    ql[gw] = 0.0
+    rho = 1.2 - 0.01 * np.arange(nzg)
+    tq, tr = _dev(ql), _dev(rho)
+    ws = torch.empty(_capi.cloud_stats_workspace_bytes(dims), dtype=torch.uint8, device="cuda")
+    out = torch.empty(nz + 4, dtype=torch.float64, device="cuda")
+    _capi.cloud_stats(dims, tr.data_ptr(), tq.data_ptr(), code, out.data_ptr(), ws.data_ptr(), D.stream())
+    got = out.cpu().numpy()
+    q = ql[gw:gw + nz].astype(np.float64)
+    assert np.array_equal(got[:nz], (q > 0).sum(axis=(1, 2)) * (1.0 / N))
+    assert got[nz] == (q > 0).any(axis=0).sum() / float(N)
+    k = np.flatnonzero((q > 0).any(axis=(1, 2)))
+    assert got[nz + 1] == ((k[0] + 0.5) * 20.0 if k.size else 99999.9)
+    assert got[nz + 2] == ((k[-1] + 0.5) * 20.0 if k.size else -99999.9)
+    lwp = (rho[:nz, None, None] * q * 20.0).sum() / N
+    assert abs(got[nz + 3] - lwp) <= (N * nz + 8) * eps * lwp
