@@ -83,19 +83,38 @@ static inline ZSplit correct_zsplit(long long plane, int nz, int gw) {
     while (plane / 64 * want < 16384 && nz / (2 * want) >= 2 * gw && want < 16) want *= 2;
     return zsplit_floor(nz, want, gw);
 }
-// The advection y pass's chunks of the ny rows and the z pass's chunks of the
-// interior levels (at least 2048 blocks, chunks of at least 32).
-static inline ZSplit advy_zsplit(int nx, int ny, int nz) {
-    const long long cols = (long long)((nx + 63) / 64) * ((nz + 3) / 4);
+// Chunks for an advection march of n levels (or rows) over `cols` blocks of
+// columns.  At least as many as give 2048 blocks with chunks of 32 or more
+// (8 wavefronts per SIMD in turn); from there the count that minimises
+// (rounds of 768 blocks, 3 per CU, what the FP64 passes' registers allow) x
+// (a chunk's length plus 4 for its start: the stencil window's loads and one
+// more face), with chunks of at least 4.  A small grid otherwise ran on a few
+// CUs (64 x 64 x 75 FP64: y pass 53 -> 19 us, z pass 75 -> 17), and a last
+// round that is mostly empty costs a chunk's whole time (fused y-z pass at 512
+// x 512 x 256: 1024 columns in 3 chunks, four full rounds, 1.58 and 1.63 ms
+// against 1.61 and 1.66 in 2).
+static inline ZSplit adv_zsplit(int n, long long cols) {
     int want = 1;
-    while (cols * want < 2048 && ny / (want * 2) >= 32) want *= 2;
-    return zsplit_ceil(ny, want);
+    while (cols * want < 2048 && n / (want * 2) >= 32) want *= 2;
+    ZSplit best = zsplit_ceil(n, want);
+    long long cost = -1;
+    for (; want <= n && (cost < 0 || n / want >= 4); ++want) {
+        const ZSplit z = zsplit_ceil(n, want);
+        const long long c = (cols * z.nch + 767) / 768 * (z.len + 4);
+        if (cost < 0 || c < cost) {
+            cost = c;
+            best = z;
+        }
+    }
+    return best;
+}
+// The advection y pass's chunks of the ny rows and the z pass's chunks of the
+// interior levels.
+static inline ZSplit advy_zsplit(int nx, int ny, int nz) {
+    return adv_zsplit(ny, (long long)((nx + 63) / 64) * ((nz + 3) / 4));
 }
 static inline ZSplit advz_zsplit(int nx, int ny, int nz) {
-    const long long cols = (long long)((nx + 63) / 64) * ((ny + 3) / 4);
-    int want = 1;
-    while (cols * want < 2048 && nz / (want * 2) >= 32) want *= 2;
-    return zsplit_ceil(nz, want);
+    return adv_zsplit(nz, (long long)((nx + 63) / 64) * ((ny + 3) / 4));
 }
 // The fused y-z advection pass: the z pass's chunks, none longer than
 // ADV_YZ_KMAX levels (the LDS copy of a chunk's level profiles holds that many).
