@@ -75,12 +75,11 @@ static inline ZSplit zsplit_floor(int n, int want, int minlen) {
     if (nch < 1) nch = 1;
     return ZSplit{nch, n / nch};
 }
-// The pressure correction's chunks of the interior levels (~16k waves; the
-// last chunk holds the top gw levels, the first the bottom gw, since the
-// boundary fill of each end reads them).
+// The pressure correction's chunks of the interior levels (~16k wavefronts of
+// 16-byte accesses, at least gw levels each).
 static inline ZSplit correct_zsplit(long long plane, int nz, int gw) {
     int want = 1;
-    while (plane / 64 * want < 16384 && nz / (2 * want) >= 2 * gw && want < 16) want *= 2;
+    while (plane / 128 * want < 16384 && nz / (2 * want) >= gw && want < 32) want *= 2;
     return zsplit_floor(nz, want, gw);
 }
 // Chunks for an advection march of n levels (or rows) over `cols` blocks of
@@ -144,18 +143,21 @@ static inline ZSplit thermo_zsplit(int nx, int ny, int nzg) {
 __device__ __forceinline__ double cfl_fold(double m, double c) {
     return (c <= 1.7976931348623157e308 && m == m) ? fmax(m, c) : __longlong_as_double(0x7ff8000000000000LL);
 }
-// Block maximum into *out by an integer atomic max: non-negative doubles
-// order like their bit patterns, and the positive quiet NaN above them all.
+// Maximum over a block of 256 into *out by an integer atomic max: non-negative
+// doubles order like their bit patterns, and the positive quiet NaN above them
+// all.  A block whose maximum is not above what *out already holds leaves it
+// alone (*out only grows).
 __device__ __forceinline__ void cfl_block_max(double m, double *out) {
-    __shared__ double red[256];
-    red[threadIdx.x] = m;
+    __shared__ double red[4];
+    for (int s = 32; s > 0; s >>= 1) m = cfl_fold(m, __shfl_down(m, s, 64));
+    if (threadIdx.x % 64 == 0) red[threadIdx.x / 64] = m;
     __syncthreads();
-    for (int s = blockDim.x / 2; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) red[threadIdx.x] = cfl_fold(red[threadIdx.x], red[threadIdx.x + s]);
-        __syncthreads();
+    if (threadIdx.x == 0) {
+        m = cfl_fold(cfl_fold(red[0], red[1]), cfl_fold(red[2], red[3]));
+        const unsigned long long b = (unsigned long long)__double_as_longlong(m);
+        if (b > __hip_atomic_load((unsigned long long *)out, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+            atomicMax((unsigned long long *)out, b);
     }
-    if (threadIdx.x == 0)
-        atomicMax((unsigned long long *)out, (unsigned long long)__double_as_longlong(red[0]));
 }
 
 // Periodic wrap for offsets smaller than the extent.

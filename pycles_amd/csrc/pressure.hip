@@ -27,8 +27,9 @@
 #include "common.h"
 
 extern int pycles_check_dims(const pycles_dims *d);
-extern int pycles_level_mean_ws(const Geo &g, const void *field, double *mean, double *partial,
-                                const double *base, int precision, hipStream_t st);
+// Partial sums of every level, MEAN_SPLITS per level (timestep.hip)
+constexpr int MEAN_SPLITS = 16;
+extern int pycles_level_partials(const Geo &g, const void *field, double *partial, int precision, hipStream_t st);
 
 struct pycles_pressure_plan {
     Geo g;
@@ -38,11 +39,14 @@ struct pycles_pressure_plan {
     int gx;          // kx columns per y-FFT block
     void *spec;      // [nz][ny][nxp] complex, field precision (columns nxh..nxp-1 unused)
     double *ck;      // Thomas segment carries: [nz / S][3][ny][nxp] (S levels per segment)
+    double *pm;      // or, with few columns, reciprocal pivots [nz][ny nxh] and
+    void *pc;        // the coefficients c' (field precision)
     void *twx;       // exp(-2 pi i m / nx), m < nx/2, interleaved (field precision)
     void *twy;
     double *kx2, *ky2, *rho_h, *dd, *a, *c;
-    double *mean, *partial, *cfl;
+    double *mean, *partial;
     int logx, logy, loggx;
+    bool thomas_lds;  // few columns: the z solve with stored pivots, in LDS
 };
 
 static int ilog2(long long n) {
@@ -117,19 +121,23 @@ __device__ __forceinline__ void dft(C2<T> *v) {
 // (0 .. N/8-1) of sequence b does the 8/R butterflies q = t + s N/8: it reads
 // x[q + r N/R], twiddles by w_N^{k r N/(Ns R)} with k = q mod Ns, transforms,
 // and writes to (q - k) R + k + r Ns.  Ns is the length of the sub-transforms
-// already combined.  All threads of the block take part (two barriers).
+// already combined.  All threads of the block take part in the two barriers;
+// those without a butterfly (act false) do nothing else.
 template <typename T, int R, bool INV>
-__device__ __forceinline__ void stockham_pass(C2<T> *buf, int S, int b, int t, int N, int Ns, const C2<T> *tw) {
+__device__ __forceinline__ void stockham_pass(C2<T> *buf, int S, int b, int t, int N, int Ns, const C2<T> *tw,
+                                              bool act) {
     constexpr int NB = 8 / R;
     const int NR = N / R, N8 = N >> 3;
     C2<T> v[NB][R];
+    if (act)
 #pragma unroll
-    for (int s = 0; s < NB; ++s) {
-        const int q = t + s * N8;
+        for (int s = 0; s < NB; ++s) {
+            const int q = t + s * N8;
 #pragma unroll
-        for (int r = 0; r < R; ++r) v[s][r] = buf[(q + r * NR) * S + b];
-    }
+            for (int r = 0; r < R; ++r) v[s][r] = buf[(q + r * NR) * S + b];
+        }
     __syncthreads();
+    if (act)
 #pragma unroll
     for (int s = 0; s < NB; ++s) {
         const int q = t + s * N8;
@@ -155,25 +163,27 @@ __device__ __forceinline__ void stockham_pass(C2<T> *buf, int S, int b, int t, i
 // sequences in buf, N = 2^logN >= 8, in natural order in and out.
 // tw[m] = exp(-2 pi i m/N), m < N.
 template <typename T, bool INV>
-__device__ void stockham_fft(C2<T> *buf, int S, int b, int t, int N, int logN, const C2<T> *tw) {
+__device__ void stockham_fft(C2<T> *buf, int S, int b, int t, int N, int logN, const C2<T> *tw, bool act = true) {
     int Ns = 1;
     const int rem = logN % 3;
     if (rem == 1) {
-        stockham_pass<T, 2, INV>(buf, S, b, t, N, Ns, tw);
+        stockham_pass<T, 2, INV>(buf, S, b, t, N, Ns, tw, act);
         Ns = 2;
     } else if (rem == 2) {
-        stockham_pass<T, 4, INV>(buf, S, b, t, N, Ns, tw);
+        stockham_pass<T, 4, INV>(buf, S, b, t, N, Ns, tw, act);
         Ns = 4;
     }
     for (int p = 0; p < logN / 3; ++p) {
-        stockham_pass<T, 8, INV>(buf, S, b, t, N, Ns, tw);
+        stockham_pass<T, 8, INV>(buf, S, b, t, N, Ns, tw, act);
         Ns *= 8;
     }
 }
 
 // ---------------------------------------------------------------------------
-// Level mean of w is computed before this kernel.  One block per 2S
-// consecutive rows (j0 .. j0+2S-1) of one level: divergence
+// The partial sums of w's levels are computed before this kernel; every
+// wavefront adds those of its level and the level below in order, and the level's first block writes the mean
+// that the correction reads and, on the last stage, clears the CFL maximum.
+// One block per 2S consecutive rows (j0 .. j0+2S-1) of one level: divergence
 // (PressureSolver.pyx:138-175, zeroed then x, y, z contributions added in that
 // order), then the forward FFT along x of the rows in pairs (row 2b as the
 // real part and row 2b+1 as the imaginary part of one complex sequence),
@@ -181,8 +191,9 @@ __device__ void stockham_fft(C2<T> *buf, int S, int b, int t, int N, int logN, c
 template <typename TS>
 __global__ __launch_bounds__(512) void div_fftx_kernel(Geo g, const TS *u, const TS *v, const TS *w,
                                                        const double *alpha0, const double *alpha0_half,
-                                                       const double *mean, TS *div_out, C2<TS> *spec,
-                                                       const C2<TS> *tw, int logx, int nxh, int nxp, int logS) {
+                                                       const double *partial, double *mean, double *cfl, TS *div_out,
+                                                       C2<TS> *spec, const C2<TS> *tw, int logx, int nxh, int nxp,
+                                                       int logS) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const int S = 1 << logS;
     C2<TS> *buf = reinterpret_cast<C2<TS> *>(smem_raw);
@@ -192,7 +203,30 @@ __global__ __launch_bounds__(512) void div_fftx_kernel(Geo g, const TS *u, const
     const int j0 = blockIdx.x << (logS + 1);
     const double ah = alpha0_half[k];
     const double a0 = alpha0[k], a0m = alpha0[k - 1];
-    const double mk = mean[k], mkm = mean[k - 1];
+    // multiplied by 1/(n0*n1) as the reference does
+    const double rn = 1.0 / (double)((long long)g.ny * g.nx);
+    double mk = 0.0, mkm = 0.0;
+    if (blockDim.x >= 2 * MEAN_SPLITS) {
+        // lanes 0..15: the partials of level k, 16..31: of level k - 1
+        const int ml = threadIdx.x % (2 * MEAN_SPLITS);
+        const double ms = partial[(long long)(ml < MEAN_SPLITS ? k : k - 1) * MEAN_SPLITS + ml % MEAN_SPLITS];
+#pragma unroll
+        for (int o = 0; o < MEAN_SPLITS; ++o) {
+            mk += __shfl(ms, o, 64);
+            mkm += __shfl(ms, MEAN_SPLITS + o, 64);
+        }
+    } else {  // blocks below half a wavefront (nx = 8 or 16 with few rows)
+        for (int o = 0; o < MEAN_SPLITS; ++o) {
+            mk += partial[(long long)k * MEAN_SPLITS + o];
+            mkm += partial[(long long)(k - 1) * MEAN_SPLITS + o];
+        }
+    }
+    mk *= rn;
+    mkm *= rn;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        mean[k] = mk;
+        if (kk == 0 && cfl) *cfl = 0.0;
+    }
     const double dxi0 = 1.0 / g.dx[0], dxi1 = 1.0 / g.dx[1], dxi2 = 1.0 / g.dx[2];
     // four cells per thread at a time: all their loads are issued before the
     // arithmetic and the stores (a store in between would hold back the
@@ -250,7 +284,7 @@ __global__ __launch_bounds__(512) void div_fftx_kernel(Geo g, const TS *u, const
     }
     __syncthreads();
     const int b = threadIdx.x & (S - 1), t = threadIdx.x >> logS;
-    stockham_fft<TS, false>(buf, S, b, t, g.nx, logx, tw);
+    stockham_fft<TS, false>(buf, S, b, t, g.nx, logx, tw, t < g.nx / 8);
     // X_a[m] = (Z[m] + conj Z[N-m]) / 2, X_b[m] = -i (Z[m] - conj Z[N-m]) / 2
     for (int q = threadIdx.x; q < nxh * S; q += blockDim.x) {
         const int m = q % nxh, pb = q / nxh;
@@ -467,6 +501,146 @@ __global__ __launch_bounds__(256, 3) void thomas_kernel(Geo g, C2<TS> *spec, dou
     }
 }
 
+// The same solve for grids with few columns, where one thread per column is one
+// dependent chain (a reciprocal and seven more FP64 operations per level and
+// sweep) on a few SIMDs.  The chain of the pivots depends on the plan only, so
+// pivot_kernel forms the reciprocal pivots m and the coefficients c' once, when
+// the plan is made, with thomas_kernel's expressions.  A block of 16 columns
+// then loads all their levels' right-hand sides, m and c' into LDS together
+// (every load in flight at once) and one wavefront runs the two sweeps, the
+// real parts on lanes 0..15 and the imaginary parts on lanes 16..31: three
+// dependent operations per level forward and two back.  The same bits.
+// 64^3 FP64: 21 -> 11.5 us, 256 x 64 x 75 FP32 26 -> 17 (holding the columns
+// in LDS without stored pivots: 19.6 and 21).
+constexpr int TL_COLS = 16, TL_U = 8;
+template <typename TS> constexpr size_t thomas_lds_bytes(int nz) {
+    return (size_t)nz * (TL_COLS * (sizeof(C2<TS>) + sizeof(double) + sizeof(TS)) + sizeof(double));
+}
+// m and c' (rounded to TS, as the forward values are) of column c = ky nxh + kx,
+// [nz][ny nxh]
+template <typename TS>
+__global__ __launch_bounds__(64) void pivot_kernel(Geo g, const double *kx2, const double *ky2, const double *rho_h,
+                                                   const double *dd, const double *a, const double *c, int nxh,
+                                                   double *pm, TS *pc) {
+    const long long ncol = (long long)g.ny * nxh;
+    const long long col = (long long)blockIdx.x * 64 + threadIdx.x;
+    if (col >= ncol) return;
+    const double kk = kx2[col % nxh] + ky2[col / nxh];
+    double sc = 0.0;
+    for (int k = 0; k < g.nz; ++k) {
+        const double b = rho_h[k] * kk - dd[k];
+        const double m = k == 0 ? rcp64(b) : rcp64(b - a[k] * sc);
+        sc = c[k] * m;
+        pm[k * ncol + col] = m;
+        pc[k * ncol + col] = (TS)sc;
+    }
+}
+template <typename TS>
+__global__ __launch_bounds__(256) void thomas_lds_kernel(Geo g, C2<TS> *spec, const double *pm, const TS *pc,
+                                                         const double *a, int nxh, int nxp) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    const int nz = g.nz;
+    double *la = reinterpret_cast<double *>(smem_raw);               // [nz]
+    double *lm = la + nz;                                            // [nz][16]
+    C2<TS> *z = reinterpret_cast<C2<TS> *>(lm + (size_t)nz * TL_COLS);  // [nz][16]
+    TS *lc = reinterpret_cast<TS *>(z + (size_t)nz * TL_COLS);       // [nz][16]
+    for (int t = threadIdx.x; t < nz; t += 256) la[t] = a[t];
+    const long long ncol = (long long)g.ny * nxh, plane = (long long)g.ny * nxp;
+    const int cl = threadIdx.x % TL_COLS, lv = threadIdx.x / TL_COLS;
+    const long long cc = (long long)blockIdx.x * TL_COLS + cl;
+    const bool live = cc < ncol;
+    const long long col = live ? cc : ncol - 1;
+    C2<TS> *sp = spec + (col / nxh) * nxp + col % nxh;
+    constexpr int LV = 256 / TL_COLS, NB = 4;
+    for (int k0 = lv; k0 < nz; k0 += NB * LV) {
+        C2<TS> q[NB];
+        double m[NB];
+        TS f[NB];
+#pragma unroll
+        for (int u = 0; u < NB; ++u) {
+            const long long k = min(k0 + u * LV, nz - 1);
+            q[u] = sp[k * plane];
+            m[u] = pm[k * ncol + col];
+            f[u] = pc[k * ncol + col];
+        }
+#pragma unroll
+        for (int u = 0; u < NB; ++u) {
+            const int k = k0 + u * LV;
+            if (k < nz) {
+                z[k * TL_COLS + cl] = q[u];
+                lm[k * TL_COLS + cl] = m[u];
+                lc[k * TL_COLS + cl] = f[u];
+            }
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < 2 * TL_COLS) {
+        TS *x = reinterpret_cast<TS *>(z) + 2 * cl + threadIdx.x / TL_COLS;  // this lane's part, level stride 2 TL_COLS
+        const double *m = lm + cl;
+        const TS *f = lc + cl;
+        double xr = 0.0;
+        // forward, a batch of TL_U levels read while the one before is worked on
+        TS q[2][TL_U];
+        double pm_[2][TL_U], pa[2][TL_U];
+        auto fetch = [&](int b, int k0) {
+#pragma unroll
+            for (int u = 0; u < TL_U; ++u) {
+                const int k = min(k0 + u, nz - 1);
+                q[b][u] = x[k * 2 * TL_COLS];
+                pm_[b][u] = m[k * TL_COLS];
+                pa[b][u] = la[k];
+            }
+        };
+        auto fwd = [&](int b, int k0) {
+#pragma unroll
+            for (int u = 0; u < TL_U; ++u)
+                if (k0 + u < nz) {
+                    xr = k0 + u == 0 ? (double)q[b][u] * pm_[b][u] : ((double)q[b][u] - pa[b][u] * xr) * pm_[b][u];
+                    x[(k0 + u) * 2 * TL_COLS] = (TS)xr;
+                }
+        };
+        fetch(0, 0);
+        for (int k0 = 0; k0 < nz; k0 += 2 * TL_U) {
+            fetch(1, k0 + TL_U);
+            fwd(0, k0);
+            fetch(0, k0 + 2 * TL_U);
+            fwd(1, k0 + TL_U);
+        }
+        // back substitution from the level below the top, whose solution is
+        // its forward value, carried unrounded
+        TS fq[2][TL_U];
+        auto bfetch = [&](int b, int k0) {
+#pragma unroll
+            for (int u = 0; u < TL_U; ++u) {
+                const int k = max(k0 - u, 0);
+                q[b][u] = x[k * 2 * TL_COLS];
+                fq[b][u] = f[k * TL_COLS];
+            }
+        };
+        auto bwd = [&](int b, int k0) {
+#pragma unroll
+            for (int u = 0; u < TL_U; ++u)
+                if (k0 - u >= 0) {
+                    xr = (double)q[b][u] - (double)fq[b][u] * xr;
+                    x[(k0 - u) * 2 * TL_COLS] = (TS)xr;
+                }
+        };
+        bfetch(0, nz - 2);
+        for (int k0 = nz - 2; k0 >= 0; k0 -= 2 * TL_U) {
+            bfetch(1, k0 - TL_U);
+            bwd(0, k0);
+            bfetch(0, k0 - 2 * TL_U);
+            bwd(1, k0 - TL_U);
+        }
+    }
+    __syncthreads();
+    // the (0,0) mode is set to zero
+    const bool zero = col == 0;
+    if (live)
+        for (int k = lv; k < nz; k += LV)
+            sp[(long long)k * plane] = zero ? C2<TS>{TS(0), TS(0)} : z[k * TL_COLS + cl];
+}
+
 // Inverse x transform of 2S rows in pairs: Z[m] = X_a[m] + i X_b[m] with the
 // Hermitian extension X[N-m] = conj X[m], one inverse FFT, real part -> row
 // 2b and imaginary part -> row 2b+1, times 1/nx, written to p at level k'+gw
@@ -528,95 +702,100 @@ __global__ __launch_bounds__(512) void ifftx_kernel(Geo g, const C2<TS> *spec, T
 }
 
 // second_order_pressure_correction (PressureSolver.pyx:83-110) after the mean
-// removal of w, then the z ghost fill of u, v (sym) and w (asym) of this
-// column, and the CFL maximum of the corrected interior.
-template <typename TS>
-__global__ __launch_bounds__(256) void correct_kernel(Geo g, TS *u, TS *v, TS *w, const TS *p, const double *mean,
-                                                      double dt, double *cfl, int kchunk) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int j = blockIdx.y;
-    // chunks of kchunk levels; the last one also takes the remainder, so
-    // every chunk holds at least kchunk >= gw levels (or the whole column)
-    const int k0 = g.gw + blockIdx.z * kchunk;
-    const int k1 = blockIdx.z + 1 == gridDim.z ? g.nz + g.gw : k0 + kchunk;
+// removal of w, with the z ghost levels of u, v (sym) and w (asym) that each
+// corrected level feeds, and the CFL maximum of the corrected interior.  V
+// consecutive columns per thread (16-byte accesses; nx is a power of two), a
+// z chunk per block row; p at level k comes from the level below's step.
+// Bound: HBM, 7 field passes; u, v and w, read and written once, through
+// non-temporal accesses.  512 x 512 x 256: FP64 764 -> 699 us (5.4 TB/s; 813
+// with ordinary accesses), FP32 378 -> 345 us; 64^3 FP64 10 -> 6.5 (one column
+// per thread and one row per block before).
+template <typename TS, int V>
+__global__ __launch_bounds__(256) void correct_kernel(Geo g, TS *u, TS *v, TS *w, const TS *p,
+                                                      const double *__restrict__ mean, double dt, double *cfl,
+                                                      int kchunk) {
+    typedef TS VT __attribute__((ext_vector_type(V)));
+    const long long e = ((long long)blockIdx.x * 256 + threadIdx.x) * V;
+    const int k0 = g.gw + blockIdx.y * kchunk;
+    const int k1 = blockIdx.y + 1 == gridDim.y ? g.nz + g.gw : k0 + kchunk;
+    const int gw = g.gw, nzg = g.nzg;
+    const long long P = g.plane;
+    auto get = [](const TS *f) { return *reinterpret_cast<const VT *>(f); };
+    auto getn = [](const TS *f) { return __builtin_nontemporal_load(reinterpret_cast<const VT *>(f)); };
+    auto put = [](TS *f, VT x) { __builtin_nontemporal_store(x, reinterpret_cast<VT *>(f)); };
     double cm = 0.0;
-    if (i < g.nx) {
-        const int ip = i + 1 == g.nx ? 0 : i + 1;
-        const int jp = j + 1 == g.ny ? 0 : j + 1;
-        const long long col = (long long)j * g.nx + i;
-        const long long ce = (long long)j * g.nx + ip;
-        const long long cn = (long long)jp * g.nx + i;
-        TS pc = p[(long long)k0 * g.plane + col];
+    if (e < P) {
+        const int i = (int)(e & (g.nx - 1));
+        const long long r = e - i;
+        const long long ce = i + V == g.nx ? r : e + V;          // the column east of the last one
+        const long long cn = r + g.nx == P ? (long long)i : e + g.nx;  // the row to the north
+        VT pc = get(p + (long long)k0 * P + e);
         // four levels at a time: all their loads before their stores (a store
         // would hold back the next level's loads, which it may alias)
         for (int kb = k0; kb < k1; kb += 4) {
-            TS uq[4], vq[4], wq[4], peq[4], pnq[4], ptq[4];
+            VT uq[4], vq[4], wq[4], pnq[4], ptq[4];
+            TS peq[4];
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const int k = min(kb + q, k1 - 1);  // a clamped duplicate past the end: loaded, not stored
-                const long long lo = (long long)k * g.plane;
-                const long long o = lo + col;
+                const long long lo = (long long)k * P;
                 peq[q] = p[lo + ce];
-                pnq[q] = p[lo + cn];
-                ptq[q] = p[o + g.plane];
-                uq[q] = u[o];
-                vq[q] = v[o];
-                wq[q] = w[o];
+                pnq[q] = get(p + lo + cn);
+                ptq[q] = get(p + lo + P + e);
+                uq[q] = getn(u + lo + e);
+                vq[q] = getn(v + lo + e);
+                wq[q] = getn(w + lo + e);
             }
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const int k = kb + q;
                 if (k >= k1) break;
-                const long long o = (long long)k * g.plane + col;
-                const TS pe = peq[q], pn = pnq[q], pt = ptq[q];
-                TS un, vn, wn;
-                if (sizeof(TS) == 8) {
-                    un = uq[q] - (pe - pc) * g.dxi[0];
-                    vn = vq[q] - (pn - pc) * g.dxi[1];
-                    const double wm = (double)wq[q] - mean[k];
-                    wn = (TS)(wm - ((double)pt - (double)pc) * g.dxi[2]);
-                } else {
-                    un = uq[q] - (pe - pc) * (TS)g.dxi[0];
-                    vn = vq[q] - (pn - pc) * (TS)g.dxi[1];
-                    wn = (TS)((double)wq[q] - mean[k]) - (pt - pc) * (TS)g.dxi[2];
+                const long long o = (long long)k * P + e;
+                const double mk = mean[k];
+                VT un, vn, wn;
+#pragma unroll
+                for (int c = 0; c < V; ++c) {
+                    const TS pcc = pc[c], pe = c + 1 < V ? pc[c + 1 < V ? c + 1 : c] : peq[q], pn = pnq[q][c], pt = ptq[q][c];
+                    if (sizeof(TS) == 8) {
+                        un[c] = uq[q][c] - (pe - pcc) * g.dxi[0];
+                        vn[c] = vq[q][c] - (pn - pcc) * g.dxi[1];
+                        const double wm = (double)wq[q][c] - mk;
+                        wn[c] = (TS)(wm - ((double)pt - (double)pcc) * g.dxi[2]);
+                    } else {
+                        un[c] = uq[q][c] - (pe - pcc) * (TS)g.dxi[0];
+                        vn[c] = vq[q][c] - (pn - pcc) * (TS)g.dxi[1];
+                        wn[c] = (TS)((double)wq[q][c] - mk) - (pt - pcc) * (TS)g.dxi[2];
+                    }
+                    if (cfl) {
+                        const double x = dt * (fabs((double)un[c]) * g.dxi[0] + fabs((double)vn[c]) * g.dxi[1] +
+                                               fabs((double)wn[c]) * g.dxi[2]);
+                        cm = cfl_fold(cm, x);
+                    }
                 }
-                u[o] = un;
-                v[o] = vn;
-                w[o] = wn;
-                if (cfl) {
-                    const double c = dt * (fabs((double)un) * g.dxi[0] + fabs((double)vn) * g.dxi[1] +
-                                           fabs((double)wn) * g.dxi[2]);
-                    cm = cfl_fold(cm, c);
+                put(u + o, un);
+                put(v + o, vn);
+                put(w + o, wn);
+                // the ghost levels this level feeds (as rk_store in advection_impl.h)
+                if (k < 2 * gw) {
+                    put(u + (long long)(2 * gw - 1 - k) * P + e, un);
+                    put(v + (long long)(2 * gw - 1 - k) * P + e, vn);
+                    if (k == gw) put(w + (long long)(gw - 1) * P + e, VT(TS(0)));
+                    if (k <= 2 * gw - 2) put(w + (long long)(2 * gw - 2 - k) * P + e, -wn);
                 }
-                pc = pt;
+                if (k >= nzg - 2 * gw) {
+                    put(u + (long long)(2 * (nzg - gw) - 1 - k) * P + e, un);
+                    put(v + (long long)(2 * (nzg - gw) - 1 - k) * P + e, vn);
+                    if (k == nzg - gw - 1) put(w + (long long)(nzg - gw) * P + e, VT(TS(0)));
+                    if (k >= nzg - 2 * gw + 1) put(w + (long long)(2 * (nzg - gw) - k) * P + e, -wn);
+                }
+                pc = ptq[q];
             }
-        }
-        // z ghost levels from the corrected boundary levels this thread wrote:
-        // the first chunk holds levels gw..2gw-1 and the last nz..nz+gw-1
-        // (each chunk has at least gw levels unless it is the whole column)
-        if (k0 == g.gw) {
-            for (int m = 0; m < g.gw; ++m) {
-                u[gidx(g, i, j, g.gw - 1 - m)] = u[gidx(g, i, j, g.gw + m)];
-                v[gidx(g, i, j, g.gw - 1 - m)] = v[gidx(g, i, j, g.gw + m)];
-            }
-            w[gidx(g, i, j, g.gw - 1)] = TS(0);
-            for (int m = 1; m < g.gw; ++m) w[gidx(g, i, j, g.gw - 1 - m)] = TS(-1.0) * w[gidx(g, i, j, g.gw - 1 + m)];
-        }
-        if (k1 == g.nz + g.gw) {
-            for (int m = 0; m < g.gw; ++m) {
-                u[gidx(g, i, j, g.nzg - g.gw + m)] = u[gidx(g, i, j, g.nzg - g.gw - 1 - m)];
-                v[gidx(g, i, j, g.nzg - g.gw + m)] = v[gidx(g, i, j, g.nzg - g.gw - 1 - m)];
-            }
-            w[gidx(g, i, j, g.nzg - g.gw)] = TS(0);
-            for (int m = 1; m < g.gw; ++m)
-                w[gidx(g, i, j, g.nzg - g.gw + m)] = TS(-1.0) * w[gidx(g, i, j, g.nzg - g.gw - m)];
         }
     }
-    if (cfl) cfl_block_max(cm, cfl);
+    // + 1e-11 as compute_cfl_max: rounding is monotonic, so adding it to every
+    // block's maximum gives the maximum plus it
+    if (cfl) cfl_block_max(cm + 1e-11, cfl);
 }
-
-__global__ void cfl_zero_kernel(double *c) { *c = 0.0; }
-__global__ void cfl_add_kernel(const double *src, double *dst) { *dst = *src + 1e-11; }
 
 // Standalone divergence (interior) in the field precision.
 template <typename TS>
@@ -719,9 +898,25 @@ extern "C" int pycles_pressure_plan_create(const pycles_dims *dims, const double
         }                                                   \
     } while (0)
     ALLOC(P->spec, nspec * cs);
+    // the z solve's form for few columns: its blocks all resident at once
     {
-        const int seg = precision == PYCLES_F64 ? thomas_seg<double>() : thomas_seg<float>();
-        ALLOC(P->ck, 3 * sizeof(double) * (size_t)(g.nz / seg + 1) * g.ny * P->nxp);
+        const size_t lds = precision == PYCLES_F64 ? thomas_lds_bytes<double>(g.nz) : thomas_lds_bytes<float>(g.nz);
+        const long long blocks = ((long long)g.ny * P->nxh + TL_COLS - 1) / TL_COLS;
+        P->thomas_lds = lds <= 160 * 1024 && blocks <= 256 * (long long)(160 * 1024 / lds) && blocks <= 2048;
+        if (P->thomas_lds && lds > 64 * 1024) {
+            const void *fn = precision == PYCLES_F64 ? (const void *)thomas_lds_kernel<double>
+                                                     : (const void *)thomas_lds_kernel<float>;
+            // the limit for every plan of this form, not this one's size
+            if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess)
+                P->thomas_lds = false;
+        }
+        if (P->thomas_lds) {
+            ALLOC(P->pm, sizeof(double) * (size_t)g.nz * g.ny * P->nxh);
+            ALLOC(P->pc, es * (size_t)g.nz * g.ny * P->nxh);
+        } else {
+            const int seg = precision == PYCLES_F64 ? thomas_seg<double>() : thomas_seg<float>();
+            ALLOC(P->ck, 3 * sizeof(double) * (size_t)(g.nz / seg + 1) * g.ny * P->nxp);
+        }
     }
     ALLOC(P->twx, (size_t)g.nx * cs);
     ALLOC(P->twy, (size_t)g.ny * cs);
@@ -732,8 +927,7 @@ extern "C" int pycles_pressure_plan_create(const pycles_dims *dims, const double
     ALLOC(P->a, nz * 8);
     ALLOC(P->c, nz * 8);
     ALLOC(P->mean, (size_t)g.nzg * 8);
-    ALLOC(P->partial, (size_t)g.nzg * 16 * 8);
-    ALLOC(P->cfl, 16);
+    ALLOC(P->partial, (size_t)g.nzg * MEAN_SPLITS * 8);
 #undef ALLOC
     hipError_t e = hipSuccess;
     if (precision == PYCLES_F64) {
@@ -757,14 +951,30 @@ extern "C" int pycles_pressure_plan_create(const pycles_dims *dims, const double
         pycles_pressure_plan_destroy(P);
         return PYCLES_ERR_HIP;
     }
+    if (P->thomas_lds) {
+        const dim3 grid((unsigned)(((long long)g.ny * P->nxh + 63) / 64));
+        if (precision == PYCLES_F64)
+            hipLaunchKernelGGL(pivot_kernel<double>, grid, dim3(64), 0, 0, g, P->kx2, P->ky2, P->rho_h, P->dd, P->a, P->c,
+                               P->nxh, P->pm, (double *)P->pc);
+        else
+            hipLaunchKernelGGL(pivot_kernel<float>, grid, dim3(64), 0, 0, g, P->kx2, P->ky2, P->rho_h, P->dd, P->a, P->c,
+                               P->nxh, P->pm, (float *)P->pc);
+        e = hipGetLastError();
+        if (e == hipSuccess) e = hipStreamSynchronize(0);  // any stream may use the plan
+        if (e != hipSuccess) {
+            pycles_set_error("pressure: pivots: %s", hipGetErrorString(e));
+            pycles_pressure_plan_destroy(P);
+            return PYCLES_ERR_HIP;
+        }
+    }
     *out = P;
     return PYCLES_OK;
 }
 
 extern "C" void pycles_pressure_plan_destroy(pycles_pressure_plan *P) {
     if (!P) return;
-    void *ptrs[] = {P->spec, P->ck, P->twx, P->twy, P->kx2, P->ky2, P->rho_h,
-                    P->dd, P->a, P->c, P->mean, P->partial, P->cfl};
+    void *ptrs[] = {P->spec, P->ck, P->pm, P->pc, P->twx, P->twy, P->kx2, P->ky2, P->rho_h,
+                    P->dd, P->a, P->c, P->mean, P->partial};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     delete P;
@@ -774,17 +984,25 @@ template <typename TS>
 static int run_pressure(pycles_pressure_plan *P, const pycles_ref *ref, void *u, void *v, void *w, void *p,
                         void *div, double dt, double *cfl_out, hipStream_t st) {
     const Geo &g = P->g;
-    int rc = pycles_level_mean_ws(g, w, P->mean, P->partial, nullptr, P->precision, st);
+    int rc = pycles_level_partials(g, w, P->partial, P->precision, st);
     if (rc) return rc;
-    // x transforms: S complex sequences (2S rows) per block, S nx/8 threads
+    // x transforms: S complex sequences (2S rows) per block, S nx/8 threads; as
+    // many sequences as 2048 points hold, fewer on grids below 2 blocks per CU.
+    // With less than four wavefronts per SIMD the divergence takes four times
+    // the threads, four cells each (16 with S nx/8 threads, in four rounds of
+    // loads and divisions); the transform's S nx/8 are the first of them.
+    // 64^3 FP64: 11.4 us and 4.8 for the means' kernel -> 7.7 for both.
     int logS = 0;
     while ((g.nx << (logS + 1)) <= 2048 && (2 << (logS + 1)) <= g.ny) ++logS;
+    while (logS > 0 && (long long)(g.ny >> (logS + 1)) * g.nz < 512 && (g.nx << logS) / 8 > 64) --logS;
     const int S = 1 << logS;
     const size_t rowsmem = sizeof(C2<TS>) * (size_t)g.nx * S;
     const int bx = S * g.nx / 8;
-    hipLaunchKernelGGL(div_fftx_kernel<TS>, dim3(g.ny / (2 * S), g.nz), dim3(bx), rowsmem, st, g, (const TS *)u,
-                       (const TS *)v, (const TS *)w, ref->alpha0, ref->alpha0_half, P->mean, (TS *)div,
-                       (C2<TS> *)P->spec, (const C2<TS> *)P->twx, P->logx, P->nxh, P->nxp, logS);
+    const long long waves = (long long)(g.ny / (2 * S)) * g.nz * ((bx + 63) / 64);
+    const int dbx = waves < 4096 && bx >= 32 && bx <= 128 ? 4 * bx : bx;
+    hipLaunchKernelGGL(div_fftx_kernel<TS>, dim3(g.ny / (2 * S), g.nz), dim3(dbx), rowsmem, st, g, (const TS *)u,
+                       (const TS *)v, (const TS *)w, ref->alpha0, ref->alpha0_half, P->partial, P->mean, cfl_out,
+                       (TS *)div, (C2<TS> *)P->spec, (const C2<TS> *)P->twx, P->logx, P->nxh, P->nxp, logS);
     PYCLES_CHECK_LAUNCH();
     const size_t ysmem = sizeof(C2<TS>) * (size_t)g.ny * P->gx;
     const dim3 ygrid((P->nxh + P->gx - 1) / P->gx, g.nz);
@@ -793,9 +1011,14 @@ static int run_pressure(pycles_pressure_plan *P, const pycles_ref *ref, void *u,
                        (const C2<TS> *)P->twy, P->logy, P->nxh, P->nxp, P->gx, P->loggx, 0);
     PYCLES_CHECK_LAUNCH();
     const long long ncol = (long long)g.ny * P->nxp;
-    hipLaunchKernelGGL((thomas_kernel<TS, thomas_seg<TS>()>), dim3((unsigned)((ncol + 255) / 256)), dim3(256),
-                       4 * sizeof(double) * (size_t)g.nz, st, g, (C2<TS> *)P->spec, P->ck, P->kx2, P->ky2,
-                       P->rho_h, P->dd, P->a, P->c, P->nxh, P->nxp);
+    if (P->thomas_lds)
+        hipLaunchKernelGGL(thomas_lds_kernel<TS>, dim3((unsigned)(((long long)g.ny * P->nxh + TL_COLS - 1) / TL_COLS)),
+                           dim3(256), thomas_lds_bytes<TS>(g.nz), st, g, (C2<TS> *)P->spec, P->pm, (const TS *)P->pc,
+                           P->a, P->nxh, P->nxp);
+    else
+        hipLaunchKernelGGL((thomas_kernel<TS, thomas_seg<TS>()>), dim3((unsigned)((ncol + 255) / 256)), dim3(256),
+                           4 * sizeof(double) * (size_t)g.nz, st, g, (C2<TS> *)P->spec, P->ck, P->kx2, P->ky2,
+                           P->rho_h, P->dd, P->a, P->c, P->nxh, P->nxp);
     PYCLES_CHECK_LAUNCH();
     hipLaunchKernelGGL(ffty_kernel<TS>, ygrid, dim3(by), ysmem, st, g, (C2<TS> *)P->spec,
                        (const C2<TS> *)P->twy, P->logy, P->nxh, P->nxp, P->gx, P->loggx, 1);
@@ -803,17 +1026,17 @@ static int run_pressure(pycles_pressure_plan *P, const pycles_ref *ref, void *u,
     hipLaunchKernelGGL(ifftx_kernel<TS>, dim3(g.ny / (2 * S), g.nz), dim3(bx), rowsmem, st, g,
                        (const C2<TS> *)P->spec, (TS *)p, (const C2<TS> *)P->twx, P->logx, P->nxh, P->nxp, logS);
     PYCLES_CHECK_LAUNCH();
-    if (cfl_out) hipLaunchKernelGGL(cfl_zero_kernel, dim3(1), dim3(1), 0, st, P->cfl);
-    // z chunks so the grid holds ~16k waves
     const ZSplit zs = correct_zsplit(g.plane, g.nz, g.gw);
-    const int nch = zs.nch, kchunk = zs.len;
-    hipLaunchKernelGGL(correct_kernel<TS>, dim3((g.nx + 255) / 256, g.ny, nch), dim3(256), 0, st, g, (TS *)u,
-                       (TS *)v, (TS *)w, (const TS *)p, P->mean, dt, cfl_out ? P->cfl : nullptr, kchunk);
+    constexpr int V = 16 / sizeof(TS);
+    const bool wide = (((uintptr_t)u | (uintptr_t)v | (uintptr_t)w | (uintptr_t)p) & 15) == 0;
+    const dim3 cgrid((unsigned)((g.plane / (wide ? V : 1) + 255) / 256), zs.nch);
+    if (wide)
+        hipLaunchKernelGGL((correct_kernel<TS, V>), cgrid, dim3(256), 0, st, g, (TS *)u, (TS *)v, (TS *)w, (const TS *)p,
+                           P->mean, dt, cfl_out, zs.len);
+    else
+        hipLaunchKernelGGL((correct_kernel<TS, 1>), cgrid, dim3(256), 0, st, g, (TS *)u, (TS *)v, (TS *)w, (const TS *)p,
+                           P->mean, dt, cfl_out, zs.len);
     PYCLES_CHECK_LAUNCH();
-    if (cfl_out) {
-        hipLaunchKernelGGL(cfl_add_kernel, dim3(1), dim3(1), 0, st, P->cfl, cfl_out);
-        PYCLES_CHECK_LAUNCH();
-    }
     return PYCLES_OK;
 }
 

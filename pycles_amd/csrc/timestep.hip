@@ -251,13 +251,12 @@ extern "C" int pycles_apply_z_bcs(const pycles_dims *dims, int nv, void *const *
 }
 
 // ---------------------------------------------------------------------------
-// Level means: partial sums per (level, split) in FP64, then a fixed-order
-// sum of the splits, so the result does not depend on scheduling.
+// Level sums: partial sums per (level, split) in FP64, in a fixed order, so the
+// result does not depend on scheduling; the projection adds the splits in order.
 #define MEAN_SPLITS 16
 
 template <typename T>
-__global__ __launch_bounds__(256) void level_partial_kernel(Geo g, const T *f, double *partial,
-                                                            const double *base) {
+__global__ __launch_bounds__(256) void level_partial_kernel(Geo g, const T *f, double *partial) {
     const int k = blockIdx.x;
     const int sp = blockIdx.y;
     const long long n = g.plane;
@@ -283,30 +282,15 @@ __global__ __launch_bounds__(256) void level_partial_kernel(Geo g, const T *f, d
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
     __syncthreads();
     if (threadIdx.x == 0) partial[(long long)k * MEAN_SPLITS + sp] = (red[0] + red[1]) + (red[2] + red[3]);
-    (void)base;
 }
 
-__global__ void level_final_kernel(Geo g, const double *partial, double *mean, const double *base) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= g.nzg) return;
-    double s = 0.0;
-    for (int sp = 0; sp < MEAN_SPLITS; ++sp) s += partial[(long long)k * MEAN_SPLITS + sp];
-    // multiply by 1/(n0*n1) as the reference does
-    double m = s * (1.0 / (double)((long long)g.ny * g.nx));
-    if (base) m += base[k];
-    mean[k] = m;
-}
-
-int pycles_level_mean_ws(const Geo &g, const void *field, double *mean, double *partial,
-                         const double *base, int precision, hipStream_t st) {
+// partial[k][MEAN_SPLITS]: the split sums of every level (pressure.hip)
+int pycles_level_partials(const Geo &g, const void *field, double *partial, int precision, hipStream_t st) {
+    const dim3 grid(g.nzg, MEAN_SPLITS);
     if (precision == PYCLES_F64)
-        hipLaunchKernelGGL(level_partial_kernel<double>, dim3(g.nzg, MEAN_SPLITS), dim3(256), 0, st, g,
-                           (const double *)field, partial, base);
+        hipLaunchKernelGGL(level_partial_kernel<double>, grid, dim3(256), 0, st, g, (const double *)field, partial);
     else
-        hipLaunchKernelGGL(level_partial_kernel<float>, dim3(g.nzg, MEAN_SPLITS), dim3(256), 0, st, g,
-                           (const float *)field, partial, base);
-    PYCLES_CHECK_LAUNCH();
-    hipLaunchKernelGGL(level_final_kernel, dim3((g.nzg + 255) / 256), dim3(256), 0, st, g, partial, mean, base);
+        hipLaunchKernelGGL(level_partial_kernel<float>, grid, dim3(256), 0, st, g, (const float *)field, partial);
     PYCLES_CHECK_LAUNCH();
     return PYCLES_OK;
 }

@@ -304,3 +304,62 @@ def test_dry_thermo_tiles(n, gw, precision):
         want = dw + (0.0 if over else wt0.astype(np.float64))
         want[nzg - 2:] = wt0[nzg - 2:]
         assert np.all(np.abs(wt.cpu().numpy().astype(np.float64) - want) <= 6e-14 * 9.80665 + (r - 1e-14) * np.abs(want))
+
+
+@pytest.mark.parametrize("n,gw,shift", [((8, 8, 5), 5, 0), ((16, 8, 9), 3, 1), ((8, 64, 2), 2, 0), ((64, 64, 64), 3, 0),
+                                        ((32, 16, 104), 3, 1), ((16, 8, 315), 3, 0), ((16, 8, 316), 3, 0),
+                                        ((256, 128, 12), 3, 0), ((512, 256, 3), 3, 1)])
+def test_projection_forms(n, gw, shift):
+    """The projection in the forms its size rules choose (few columns with
+    stored pivots in LDS, up to 315 FP64 levels; blocks of less than half a
+    wavefront; few and many sequences per block) and off a 16-byte boundary (shift), FP64 against the
+    oracle: 1e-12 of each field's maximum, as test_pressure_parity.  The CFL
+    maximum is exact for the velocities that come back."""
+    import torch
+    from oracle import oracle as O
+    from pycles_amd import _capi
+    from pycles_amd import _device as D
+    nx, ny, nz = n
+    nzg, N = nz + 2 * gw, nx * ny * (nz + 2 * gw)
+    dx = (50.0, 60.0, 20.0)
+    rng = np.random.default_rng(nx + nz)
+    alpha = 0.8 + 0.5 * np.arange(nzg) / nzg
+    half = alpha - 0.004
+    prof = {"rho0": 1.0 / alpha, "rho0_half": 1.0 / half, "alpha0": alpha, "alpha0_half": half,
+            "p0": 1e5 - np.arange(nzg), "p0_half": 1e5 - np.arange(nzg)}
+    oref = O.Ref(prof["p0"], prof["p0_half"], alpha, half, prof["rho0"], prof["rho0_half"])
+    dp = {k: _dev(v) for k, v in prof.items()}
+    ref = _capi.Ref(*[dp[k].data_ptr() for k in ("rho0", "rho0_half", "alpha0", "alpha0_half", "p0", "p0_half")])
+    f = {k: rng.standard_normal((nzg, ny, nx)) for k in "uvw"}
+    for a, sgn in ((f["u"], 1), (f["v"], 1), (f["w"], -1)):
+        if sgn > 0:
+            a[:gw], a[nzg - gw:] = a[gw:2 * gw][::-1], a[nzg - 2 * gw:nzg - gw][::-1]
+        else:
+            a[gw - 1] = a[nzg - gw] = a[nzg - gw - 1] = 0.0
+    sim = O.OracleSimulation(O.make_dims(nx, ny, nz, gw, *dx), oref, False, None)
+    for k in "uvw":
+        sim.pv(k)[...] = np.pad(f[k].transpose(2, 1, 0), ((gw, gw), (gw, gw), (0, 0)), mode="wrap")
+    sim.pressure_update()
+    buf = torch.zeros(3 * N + 4, dtype=torch.float64, device="cuda")
+    for q, k in enumerate("uvw"):
+        buf[shift + q * N:shift + (q + 1) * N] = _dev(f[k]).reshape(-1)
+    ptr = [buf.data_ptr() + 8 * (shift + q * N) for q in range(3)]
+    p, div = (torch.zeros((nzg, ny, nx), dtype=torch.float64, device="cuda") for _ in range(2))
+    cfl = torch.full((1,), 1e30, dtype=torch.float64, device="cuda")
+    dims = _dims(n, gw, dx)
+    plan = _capi.PressurePlan(dims, prof["rho0"].ctypes.data, prof["rho0_half"].ctypes.data, D.F64)
+    plan.update(ref, *ptr, p.data_ptr(), div.data_ptr(), 0.75, cfl.data_ptr(), D.stream())
+    got = buf[shift:shift + 3 * N].cpu().numpy().reshape(3, nzg, ny, nx)
+
+    def err(a, name, dv=False):
+        b = np.asarray((sim.dv[name] if dv else sim.pv(name)))[gw:-gw, gw:-gw].transpose(2, 1, 0)
+        return np.abs(a - b).max() / np.abs(b).max()
+
+    for q, k in enumerate("uvw"):
+        assert err(got[q], k) <= 1e-12, k
+    assert err(p.cpu().numpy(), "dynamic_pressure", True) <= 1e-12
+    sl = slice(gw, gw + nz)
+    odiv = np.asarray(sim.dv["divergence"])[gw:-gw, gw:-gw, gw:-gw].transpose(2, 1, 0)
+    assert np.abs(div.cpu().numpy()[sl] - odiv).max() <= 1e-12 * np.abs(odiv).max()
+    c = 0.75 * ((np.abs(got[0, sl]) * (1.0 / dx[0]) + np.abs(got[1, sl]) * (1.0 / dx[1])) + np.abs(got[2, sl]) * (1.0 / dx[2]))
+    assert float(cfl[0]) == c.max() + 1e-11
