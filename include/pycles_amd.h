@@ -250,6 +250,9 @@ int pycles_apply_z_bcs(const pycles_dims *dims, int nv, void *const *values,
  * device array of nzg entries (every level, ghosts included). */
 int pycles_level_mean(const pycles_dims *dims, const void *field, double *mean, int precision,
                       void *stream);
+/* pycles_level_mean of nv (1..8) fields in one call: means[v][nzg]. */
+int pycles_level_means(const pycles_dims *dims, int nv, const void *const *fields, double *means, int precision,
+                       void *stream);
 /* compute_cfl_max (TimeStepping.pyx:222-263) into one FP64 device value
  * (max over interior of dt*(|u|/dx+|v|/dy+|w|/dz), plus 1e-11).  A NaN or
  * infinite velocity makes the value NaN (the reference's fmax would drop a

@@ -26,9 +26,7 @@ from . import thermo_host as H
 def _means(Gr, PV, names, dev):
     """Level means of the stored fields (FP64 [len(names)][nzg])."""
     out = torch.empty((len(names), Gr.dims.nzg), dtype=torch.float64, device=dev)
-    dims = D.dims_of(Gr)
-    for q, n in enumerate(names):
-        _capi.level_mean(dims, PV.ptr(n), out[q].data_ptr(), PV.precision, D.stream())
+    _capi.level_means(D.dims_of(Gr), [PV.ptr(n) for n in names], out.data_ptr(), PV.precision, D.stream())
     return out
 
 

@@ -83,6 +83,7 @@ cdef extern from "pycles_amd.h":
                          int precision, int zero_tendencies, void *stream)
     int pycles_apply_z_bcs(const pycles_dims *dims, int nv, void *const *values,
                            const double *bc_type, int precision, void *stream)
+    int pycles_level_means(const pycles_dims *, int, const void *const *, double *, int, void *) nogil
     int pycles_level_mean(const pycles_dims *dims, const void *field, double *mean, int precision,
                           void *stream)
     int pycles_cfl_max(const pycles_dims *dims, const void *u, const void *v, const void *w,
@@ -355,6 +356,16 @@ def apply_z_bcs(Dims dims, values, bc_type, int precision, stream):
 
 def level_mean(Dims dims, field, mean, int precision, stream):
     _check(pycles_level_mean(&dims.d, _p(field), <double *> _p(mean), precision, _p(stream)))
+
+
+def level_means(Dims dims, fields, means, int precision, stream):
+    cdef const void *f[8]
+    cdef int nv = len(fields)
+    if nv > 8:
+        raise ValueError("level_means: at most 8 fields")
+    for q in range(nv):
+        f[q] = _p(fields[q])
+    _check(pycles_level_means(&dims.d, nv, f, <double *> _p(means), precision, _p(stream)))
 
 
 def cfl_max(Dims dims, u, v, w, double dt, out, int precision, stream):

@@ -295,21 +295,66 @@ int pycles_level_partials(const Geo &g, const void *field, double *partial, int 
     return PYCLES_OK;
 }
 
-// Standalone entry: one block per level (no workspace needed).
+// Standalone entries: one block per level and field (no workspace needed).
+// Each thread adds its cells in order, eight loads ahead of their additions,
+// then the block's sums in a fixed tree.  Bound: latency (a launch and one
+// round of loads) on small planes: one call for the five prognostic fields of
+// 64 x 64 x 81 levels instead of five,
+// 4 us against 5 x 6.
+struct MeanPack {
+    const void *f[8];
+};
 template <typename T>
-__global__ __launch_bounds__(256) void level_mean_kernel(Geo g, const T *f, double *mean) {
-    const int k = blockIdx.x;
-    const T *row = f + (long long)k * g.plane;
+__global__ __launch_bounds__(256) void level_mean_kernel(Geo g, MeanPack pk, double *mean) {
+    constexpr int U = 8, B = 256;
+    const int k = blockIdx.x, v = blockIdx.y;
+    const T *row = (const T *)pk.f[v] + (long long)k * g.plane;
     double acc = 0.0;
-    for (long long c = threadIdx.x; c < g.plane; c += blockDim.x) acc += (double)row[c];
-    __shared__ double red[256];
+    long long c = threadIdx.x;
+    for (; c + (U - 1) * B < g.plane; c += U * B) {
+        T x[U];
+#pragma unroll
+        for (int q = 0; q < U; ++q) x[q] = row[c + q * B];
+#pragma unroll
+        for (int q = 0; q < U; ++q) acc += (double)x[q];
+    }
+    for (; c < g.plane; c += B) acc += (double)row[c];
+    __shared__ double red[B];
     red[threadIdx.x] = acc;
     __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-        __syncthreads();
+    if (threadIdx.x < 128) red[threadIdx.x] += red[threadIdx.x + 128];
+    __syncthreads();
+    if (threadIdx.x < 64) {
+        double s = red[threadIdx.x] + red[threadIdx.x + 64];
+        for (int o = 32; o > 0; o >>= 1) s += __shfl_down(s, o, 64);
+        if (threadIdx.x == 0) mean[(long long)v * g.nzg + k] = s * (1.0 / (double)((long long)g.ny * g.nx));
     }
-    if (threadIdx.x == 0) mean[k] = red[0] * (1.0 / (double)((long long)g.ny * g.nx));
+}
+
+extern "C" int pycles_level_means(const pycles_dims *dims, int nv, const void *const *fields, double *means,
+                                  int precision, void *stream) {
+    int rc = pycles_check_dims(dims);
+    if (rc) return rc;
+    if (nv < 1 || nv > 8 || !fields || !means || (precision != PYCLES_F64 && precision != PYCLES_F32)) {
+        pycles_set_error("level_means: bad arguments");
+        return PYCLES_ERR_ARG;
+    }
+    MeanPack pk;
+    for (int v = 0; v < 8; ++v) {
+        pk.f[v] = v < nv ? fields[v] : nullptr;
+        if (v < nv && !pk.f[v]) {
+            pycles_set_error("level_means: NULL field %d", v);
+            return PYCLES_ERR_ARG;
+        }
+    }
+    Geo g = make_geo(dims);
+    hipStream_t st = (hipStream_t)stream;
+    if (precision == PYCLES_F64)
+        hipLaunchKernelGGL(level_mean_kernel<double>, dim3(g.nzg, nv), dim3(256), 0, st, g, pk, means);
+    else
+        hipLaunchKernelGGL(level_mean_kernel<float>, dim3(g.nzg, nv), dim3(256), 0, st, g, pk, means);
+    PYCLES_CHECK_LAUNCH();
+    return PYCLES_OK;
 }
 
 extern "C" int pycles_level_mean(const pycles_dims *dims, const void *field, double *mean, int precision,
@@ -320,14 +365,7 @@ extern "C" int pycles_level_mean(const pycles_dims *dims, const void *field, dou
         pycles_set_error("level_mean: bad arguments");
         return PYCLES_ERR_ARG;
     }
-    Geo g = make_geo(dims);
-    hipStream_t st = (hipStream_t)stream;
-    if (precision == PYCLES_F64)
-        hipLaunchKernelGGL(level_mean_kernel<double>, dim3(g.nzg), dim3(256), 0, st, g, (const double *)field, mean);
-    else
-        hipLaunchKernelGGL(level_mean_kernel<float>, dim3(g.nzg), dim3(256), 0, st, g, (const float *)field, mean);
-    PYCLES_CHECK_LAUNCH();
-    return PYCLES_OK;
+    return pycles_level_means(dims, 1, &field, mean, precision, stream);
 }
 
 // ---------------------------------------------------------------------------

@@ -363,3 +363,26 @@ def test_projection_forms(n, gw, shift):
     assert np.abs(div.cpu().numpy()[sl] - odiv).max() <= 1e-12 * np.abs(odiv).max()
     c = 0.75 * ((np.abs(got[0, sl]) * (1.0 / dx[0]) + np.abs(got[1, sl]) * (1.0 / dx[1])) + np.abs(got[2, sl]) * (1.0 / dx[2]))
     assert float(cfl[0]) == c.max() + 1e-11
+
+
+@pytest.mark.parametrize("n", [(3, 5, 4), (64, 64, 6), (45, 47, 5), (160, 130, 2)])
+@pytest.mark.parametrize("precision", ["f64", "f32"])
+def test_level_means_tiles(n, precision):
+    """Level means of several fields in one call: bitwise the one-field calls',
+    and numpy's to N eps of the mean magnitude; planes below, at and beyond
+    whole batches of a block's loads."""
+    import torch
+    from pycles_amd import _capi
+    from pycles_amd import _device as D
+    code = D.precision_code(precision)
+    nzg, N = n[2] + 4, n[0] * n[1]
+    rng = np.random.default_rng(2)
+    f = rng.standard_normal((3, nzg, n[1], n[0])).astype(np.float64 if precision == "f64" else np.float32)
+    t = _dev(f)
+    many, one = (torch.full((3, nzg), 9.0, dtype=torch.float64, device="cuda") for _ in range(2))
+    _capi.level_means(_dims(n, 2), [t[q].data_ptr() for q in range(3)], many.data_ptr(), code, D.stream())
+    for q in range(3):
+        _capi.level_mean(_dims(n, 2), t[q].data_ptr(), one[q].data_ptr(), code, D.stream())
+    assert torch.equal(many, one)
+    d = f.astype(np.float64)
+    assert np.all(np.abs(many.cpu().numpy() - d.mean(axis=(2, 3))) <= (N + 8) * np.finfo(np.float64).eps * np.abs(d).mean(axis=(2, 3)))
