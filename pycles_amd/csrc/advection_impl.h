@@ -105,6 +105,10 @@ struct PolicyF64 {
     // waves per SIMD the z pass is held to (<= 168 VGPRs): its stage-2 form
     // otherwise takes 171 and runs 2 waves
     static constexpr int kZWaves = 3;
+    static constexpr bool kXVec = true;  // the x pass by vectors (adv_xv), where the rows allow it
+    static constexpr int kXCells = 2;    // its cells per thread, one 16-byte access
+    static constexpr int kXThreads = 512;
+    static constexpr int kXWaves5 = 4;     // waves per SIMD it is held to at WENO5 (128 VGPRs)
     template <int O, bool BV>
     static __device__ __forceinline__ SFlux scal_flux(const TC *win, const double *, TC U, double rho) {
         return upwind_flux<O, double>(win, U, rho);
@@ -154,6 +158,7 @@ struct PolicyF32 {
     static constexpr bool kFuseYZ = true;  // y and z passes fused (WENO5)
     static constexpr int kYZWaves = 3;     // waves per SIMD of the fused pass (its LDS allows 3 blocks per CU)
     static constexpr int kZWaves = 1;      // the z pass's registers as the compiler allocates them
+    static constexpr bool kXVec = false;   // the x pass stays the row-staged kernel
     template <int O, bool BV>
     static __device__ __forceinline__ SFlux scal_flux(const TC *win, const double *bwin, TC U, double rho) {
         constexpr int R = Interp<O, float>::R;
@@ -1250,6 +1255,204 @@ __global__ __launch_bounds__(256) void adv_x(Geo g, Prof pr, Fields fl) {
     }
 }
 
+// -------------------------------------------------------------------------
+// x pass for rows of whole vectors (nx a multiple of C = P::kXCells, fields on
+// 16-byte boundaries): C consecutive cells per thread, nx / C threads per row,
+// whole rows per block.  Each thread loads the vectors that its faces' windows
+// reach straight into registers (its own, NL to the left and NR to the right,
+// wrapped; the neighbours' come from the vector cache), computes the C faces
+// to the right of its cells and takes the face to the left of them from the
+// thread to the left through LDS: one barrier, no staged rows, no flux rows,
+// and one address per vector instead of one per cell.  The row-staged kernel
+// above spends a third of its instructions on staging and addresses.
+template <class TS, int C> struct XVec {
+    typedef TS type __attribute__((ext_vector_type(C)));
+};
+// accesses of C cells in pieces of 16 bytes
+template <class TS, int C>
+__device__ __forceinline__ void xload(const TS *p, unsigned off, TS *x) {
+    constexpr int W = 16 / sizeof(TS) < C ? 16 / sizeof(TS) : C;
+#pragma unroll
+    for (int q = 0; q < C; q += W) {
+        const auto v = *reinterpret_cast<const typename XVec<TS, W>::type *>(at(const_cast<TS *>(p), off + q));
+#pragma unroll
+        for (int e = 0; e < W; ++e) x[q + e] = v[e];
+    }
+}
+template <class TS, int C>
+__device__ __forceinline__ void xstore(TS *p, unsigned off, const TS *x) {
+    constexpr int W = 16 / sizeof(TS) < C ? 16 / sizeof(TS) : C;
+#pragma unroll
+    for (int q = 0; q < C; q += W) {
+        typename XVec<TS, W>::type v;
+#pragma unroll
+        for (int e = 0; e < W; ++e) v[e] = x[q + e];
+        *reinterpret_cast<typename XVec<TS, W>::type *>(at(p, off + q)) = v;
+    }
+}
+
+// The face to be exchanged is evaluated before the barrier and the others after
+// it, next to their divergences, which keeps the fluxes' registers short-lived
+// (at WENO5 4 waves per SIMD; all faces first, with their loads a field ahead
+// of their use, took 3 and 10% more time).  PART: the last block has rows
+// beyond ny (they work on row 0 and store nothing).
+// FP64 only: 256 x 256 x 128 WENO5 349 -> 252 us, 64^3 15 -> 11.5.  In FP32 it
+// gained 5% (750 -> 715 us at 512 x 512 x 256), but multiply-adds contracted in
+// other places than in the staged kernel move the velocities' last bits, which
+// the entropy's tendency (s div(rho u), thousands of times the net tendency in
+// each direction) amplifies to 3e-5 of its deviations after a step.
+template <class P, int SO, int MO, int NSC, bool MOM, bool PART>
+__global__ __launch_bounds__(P::kXThreads, SO == 5 && MO == 5 ? P::kXWaves5 : 1) void adv_xv(Geo g, Prof pr, Fields fl, int nt,
+                                                                                     int rows) {
+    using TS = typename P::TS;
+    using TC = typename P::TC;
+    constexpr int C = P::kXCells;
+    constexpr int RS = Interp<SO, TC>::R, RM = Interp<MO, TC>::R;
+    constexpr int RX = (MOM && RM > RS) || NSC == 0 ? RM : RS;  // widest window
+    constexpr int NL = (RX - 1 + C - 1) / C, NR = (RX + C - 1) / C;
+    constexpr int NC = 2 * (RM - 1);
+    constexpr int NF = NSC + (MOM ? 3 : 0);
+    constexpr int NS = NSC > 0 ? NSC : 1;
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    TC *edge = reinterpret_cast<TC *>(smem_raw);  // [NF][blockDim.x]: each thread's last face
+    const uint3 tile = xcd_tile<0>();  // XCD bands of rows in y
+    const int tid = threadIdx.x, B = blockDim.x;
+    const int rr = tid / nt, t = tid - rr * nt;
+    const int jr = tile.x * rows + rr;
+    const int j = !PART || jr < g.ny ? jr : 0;
+    const int k = tile.y + g.gw;
+    const unsigned plane = (unsigned)g.plane;
+    const unsigned row = ((unsigned)k * g.ny + j) * g.nx;
+    const bool tzero = fl.tzero != 0;
+    const TS *pu = (const TS *)fl.q[VU];
+    auto field = [](int f) { return f < NSC ? f : VU + (f - NSC); };
+    // offsets of this thread's vectors, NL to the left to NR to the right
+    unsigned off[NL + 1 + NR];
+#pragma unroll
+    for (int n = 0; n < NL + 1 + NR; ++n) off[n] = row + (unsigned)wrapi(t + n - NL, nt) * C;
+    const unsigned o = off[NL];
+    const double rh = pr.rho0_half[k], r0 = pr.rho0[k], ah = pr.alpha0_half[k], a0 = pr.alpha0[k];
+    const double dxi = g.dxi[0];
+    constexpr int NX = C * (NL + 1 + NR), X0 = C * NL;  // x[X0 + c]: cell C t + c
+    // the vectors of one field that windows of half-width R reach
+    auto window = [&](const void *p, TS *x, auto rc) {
+        constexpr int R = decltype(rc)::value;
+        constexpr int L = (R - 1 + C - 1) / C, U = (R + C - 1) / C;
+#pragma unroll
+        for (int n = NL - L; n <= NL + U; ++n) xload<TS, C>((const TS *)p, off[n], x + n * C);
+    };
+    std::integral_constant<int, RS> cs;
+    std::integral_constant<int, RM> cm;
+    // u: its own window with the momentum; otherwise the cells' values and the
+    // one to the left (the scalars' advecting velocity)
+    TS xu[NX], xs[NS][NX], xv[NX], xw[NX];
+    window(pu, xu, std::integral_constant<int, MOM ? RM : 2>{});
+    // u centred along y and z, for the v and w fluxes
+    TS qy[NC][C], qz[NC][C];
+    if (MOM) {
+#pragma unroll
+        for (int m = 0; m < NC; ++m) {
+            const int d = m - (RM - 2);
+            if (d == 0) {
+#pragma unroll
+                for (int e = 0; e < C; ++e) qy[m][e] = qz[m][e] = xu[X0 + e];
+                continue;
+            }
+            xload<TS, C>(pu, o + (wrapi(j + d, g.ny) - j) * g.nx, qy[m]);
+            xload<TS, C>(pu, o + d * (int)plane, qz[m]);
+        }
+    }
+    // the tendencies the pass must read: w's, which thermodynamics wrote, and
+    // the others unless they are known to be zero
+    TS told[NF > 0 ? NF : 1][C] = {};
+    if (!tzero) {
+#pragma unroll
+        for (int f = 0; f < NF - (MOM ? 1 : 0); ++f) xload<TS, C>((const TS *)fl.t[field(f)], o, told[f]);
+    }
+    if (MOM) xload<TS, C>((const TS *)fl.t[VW], o, told[NF - 1]);
+    if (NSC > 0) window(fl.q[0], xs[0], cs);
+    else window(fl.q[VV], xv, cm);
+    TC uy[C], uz[C];
+    if (MOM) {
+#pragma unroll
+        for (int e = 0; e < C; ++e) {
+            TC q[NC];
+#pragma unroll
+            for (int m = 0; m < NC; ++m) q[m] = (TC)qy[m][e];
+            uy[e] = Interp<MO, TC>::centred(q);
+#pragma unroll
+            for (int m = 0; m < NC; ++m) q[m] = (TC)qz[m][e];
+            uz[e] = Interp<MO, TC>::centred(q);
+        }
+    }
+    double bw[NS][1];
+#pragma unroll
+    for (int sc = 0; sc < NSC; ++sc) bw[sc][0] = P::kBase ? (fl.base[sc] ? fl.base[sc][k] : 0.0) : 0.0;
+    // the faces to the right of this thread's cells
+    TC F[NF > 0 ? NF : 1][C];
+    auto scalar = [&](auto scc, int lo, int hi) {
+        constexpr int sc = decltype(scc)::value;
+#pragma unroll
+        for (int e = 0; e < C; ++e)
+            if (e >= lo && e < hi)
+                F[sc][e] = P::x_keep(P::template scal_flux<SO, false>(xs[sc] + X0 + e - (RS - 1), bw[sc], xu[X0 + e], rh));
+    };
+    auto momentum = [&](int lo, int hi) {  // advected component u, v, w
+#pragma unroll
+        for (int e = 0; e < C; ++e)
+            if (e >= lo && e < hi) {
+                const TC U = Interp<MO, TC>::centred(xu + X0 + e - (RM - 2));
+                F[NSC][e] = P::template mom_flux<MO>(xu + X0 + e - (RM - 1), U, rh);
+                F[NSC + 1][e] = P::template mom_flux<MO>(xv + X0 + e - (RM - 1), uy[e], rh);
+                F[NSC + 2][e] = P::template mom_flux<MO>(xw + X0 + e - (RM - 1), uz[e], r0);
+            }
+    };
+    constexpr int E0 = C - 1;  // the face to be exchanged
+    if constexpr (NSC > 1) window(fl.q[1], xs[1], cs);
+    else if constexpr (NSC > 0 && MOM) window(fl.q[VV], xv, cm);
+    if constexpr (NSC > 0) {
+        scalar(std::integral_constant<int, 0>{}, E0, C);
+    }
+    if constexpr (NSC > 1) {
+        if (MOM) window(fl.q[VV], xv, cm);
+        scalar(std::integral_constant<int, 1>{}, E0, C);
+    }
+    if constexpr (MOM) {
+        window(fl.q[VW], xw, cm);
+        momentum(E0, C);
+    }
+#pragma unroll
+    for (int f = 0; f < NF; ++f) edge[f * B + tid] = F[f][C - 1];
+    __syncthreads();
+    if constexpr (E0 > 0) {
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (NSC > 0) scalar(std::integral_constant<int, 0>{}, 0, E0);
+        if constexpr (NSC > 1) scalar(std::integral_constant<int, 1>{}, 0, E0);
+        if constexpr (MOM) momentum(0, E0);
+    }
+    const int tl = t == 0 ? tid + nt - 1 : tid - 1;
+    TS out[NF > 0 ? NF : 1][C];
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+        TC fp = edge[f * B + tl];
+#pragma unroll
+        for (int e = 0; e < C; ++e) {
+            TS d;
+            if (f < NSC)
+                d = P::x_scal_div(F[f][e], fp, xu[X0 + e], xu[X0 + e - 1], ah, dxi, bw[f < NSC ? f : 0][0] * rh);
+            else
+                d = P::mom_div(F[f][e], fp, f == NSC + 2 ? a0 : ah, dxi);
+            fp = F[f][e];
+            // 0 - d when the tendency is zero on entry (same bits as adding to 0)
+            out[f][e] = told[f][e] - d;
+        }
+    }
+    if (!PART || jr < g.ny) {
+#pragma unroll
+        for (int f = 0; f < NF; ++f) xstore<TS, C>((TS *)fl.t[field(f)], o, out[f]);
+    }
+}
+
 template <class P, int SO, int MO, int NSC, bool MOM>
 size_t x_smem_bytes(int nx, bool tzero) {
     return XLayout<P, SO, MO, NSC, MOM>::words(nx, tzero) * sizeof(typename P::TC);
@@ -1271,9 +1474,38 @@ int launch(const Geo &g, const Prof &pr, const Fields &fl, hipStream_t st) {
             return PYCLES_ERR_UNSUPPORTED;
         }
     }
-    int bx = g.nx >= 256 ? 256 : ((g.nx + 63) / 64) * 64;
     if (fl.passes & 1) {
-        hipLaunchKernelGGL((adv_x<P, SO, MO, NSC, MOM>), dim3(g.ny, g.nz), dim3(bx), smem, st, g, pr, fl);
+        bool vec = false;
+        if constexpr (P::kXVec) {
+            // whole vectors per row, every row of every array on a 16-byte boundary
+            constexpr int C = P::kXCells;
+            const int nt = g.nx / C;
+            vec = g.nx % C == 0 && nt <= P::kXThreads && nt >= 3;
+            for (int f = 0; f < 5; ++f)
+                if (f < NSC || f >= VU) vec = vec && (((uintptr_t)fl.q[f] | (uintptr_t)fl.t[f]) & 15) == 0;
+            if (vec) {
+                // about 256 threads of whole rows; a row count that divides ny
+                // where that costs no more than half of them
+                int rows = 256 / nt > 0 ? 256 / nt : 1;
+                if (rows > g.ny) rows = g.ny;
+                for (int r = rows; r > 0 && 2 * r >= rows; --r)
+                    if (g.ny % r == 0) {
+                        rows = r;
+                        break;
+                    }
+                constexpr int NF = NSC + (MOM ? 3 : 0);
+                const dim3 grid((g.ny + rows - 1) / rows, g.nz), blk(rows * nt);
+                const size_t lds = (size_t)NF * rows * nt * sizeof(typename P::TC);
+                if (g.ny % rows != 0)
+                    hipLaunchKernelGGL((adv_xv<P, SO, MO, NSC, MOM, true>), grid, blk, lds, st, g, pr, fl, nt, rows);
+                else
+                    hipLaunchKernelGGL((adv_xv<P, SO, MO, NSC, MOM, false>), grid, blk, lds, st, g, pr, fl, nt, rows);
+            }
+        }
+        if (!vec) {
+            const int bx = g.nx >= 256 ? 256 : ((g.nx + 63) / 64) * 64;
+            hipLaunchKernelGGL((adv_x<P, SO, MO, NSC, MOM>), dim3(g.ny, g.nz), dim3(bx), smem, st, g, pr, fl);
+        }
         PYCLES_CHECK_LAUNCH();
     }
     // y and z fused (WENO5 with momentum and scalars), z-chunked like the z pass

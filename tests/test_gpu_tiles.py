@@ -386,3 +386,63 @@ def test_level_means_tiles(n, precision):
     assert torch.equal(many, one)
     d = f.astype(np.float64)
     assert np.all(np.abs(many.cpu().numpy() - d.mean(axis=(2, 3))) <= (N + 8) * np.finfo(np.float64).eps * np.abs(d).mean(axis=(2, 3)))
+
+
+@pytest.mark.parametrize("n,orders", [((12, 12, 6), (5, 5)), ((20, 11, 7), (9, 5)), ((24, 10, 6), (9, 9)), ((68, 13, 6), (7, 7)),
+                                      ((64, 37, 5), (5, 5)), ((1024, 10, 5), (5, 5)), ((1032, 10, 5), (9, 9)),
+                                      ((2048, 10, 5), (9, 9)),
+                                      ((22, 10, 5), (9, 9)), ((21, 10, 5), (5, 5))])
+@pytest.mark.parametrize("moist,shift", [(True, 0), (False, 0), (True, 1)])
+def test_advection_x_forms_bitwise(n, orders, moist, shift):
+    """FP64 tendencies, bitwise against the oracle, over the x pass's forms:
+    rows of whole vectors (one block of several rows, rows that do and do not
+    divide ny, one row per block, rows beyond its limit), odd rows and fields
+    off a 16-byte boundary (shift); tendencies zero on entry and accumulated."""
+    import torch
+    from oracle import oracle as O
+    from pycles_amd import _capi
+    from pycles_amd import _device as D
+    nx, ny, nz = n
+    gw = (max(orders) + 1) // 2
+    nzg, N = nz + 2 * gw, nx * ny * (nz + 2 * gw)
+    dx = (50.0, 60.0, 20.0)
+    rng = np.random.default_rng(nx * ny)
+    alpha = 0.8 + 0.3 * np.arange(nzg) / nzg
+    half = alpha - 0.004
+    prof = {"rho0": 1.0 / alpha, "rho0_half": 1.0 / half, "alpha0": alpha, "alpha0_half": half, "p0": alpha, "p0_half": alpha}
+    oref = O.Ref(prof["p0"], prof["p0_half"], alpha, half, prof["rho0"], prof["rho0_half"])
+    dp = {k: _dev(v) for k, v in prof.items()}
+    ref = _capi.Ref(*[dp[k].data_ptr() for k in ("rho0", "rho0_half", "alpha0", "alpha0_half", "p0", "p0_half")])
+    names = ["u", "v", "w", "s"] + (["qt"] if moist else [])
+    f = {k: rng.standard_normal((nzg, ny, nx)) for k in names}
+    t0 = {k: rng.standard_normal((nzg, ny, nx)) for k in names}
+    lt = O.Lookup(np.linspace(100.0, 380.0, 16), np.linspace(1.0, 2.0, 16)) if moist else None
+    buf = torch.zeros(2 * len(names) * N + 4, dtype=torch.float64, device="cuda")
+
+    def slot(q):
+        return buf[shift + q * N:shift + (q + 1) * N]
+
+    for zero in (0, 1):
+        sim = O.OracleSimulation(O.make_dims(nx, ny, nz, gw, *dx), oref, moist, lt, scalar_order=orders[0],
+                                 momentum_order=orders[1])
+        for q, k in enumerate(names):
+            start = t0[k] if k == "w" or not zero else np.zeros_like(t0[k])
+            sim.pv(k)[...] = np.pad(f[k].transpose(2, 1, 0), ((gw, gw), (gw, gw), (0, 0)), mode="wrap")
+            sim.pt(k)[...] = np.pad(start.transpose(2, 1, 0), ((gw, gw), (gw, gw), (0, 0)), mode="wrap")
+            slot(q).copy_(_dev(f[k]).reshape(-1))
+            slot(len(names) + q).copy_(_dev(t0[k]).reshape(-1))  # stale where zero: to be replaced
+        sim.scalar_advection_update()
+        sim.momentum_advection_update()
+        ptr = [slot(q).data_ptr() for q in range(2 * len(names))]
+        v, t = ptr[:len(names)], ptr[len(names):]
+        if nx == 2048:
+            # rows whose staged form exceeds the LDS are refused whatever the form
+            with pytest.raises(_capi.PyclesError, match="does not fit in LDS"):
+                _capi.advection(_dims(n, gw, dx), ref, v[:3], t[:3], v[3:], t[3:], None, *orders, D.F64, D.stream(), 0)
+            return
+        _capi.advection(_dims(n, gw, dx), ref, v[:3], t[:3], v[3:], t[3:], None, *orders, D.F64, D.stream(),
+                        _capi.ADV_TEND_ZERO if zero else 0)
+        for q, k in enumerate(names):
+            got = slot(len(names) + q).cpu().numpy().reshape(nzg, ny, nx)[gw:-gw]
+            want = np.asarray(sim.pt(k))[gw:-gw, gw:-gw, gw:-gw].transpose(2, 1, 0)
+            assert np.array_equal(got, want), (k, zero, np.abs(got - want).max())
