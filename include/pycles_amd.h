@@ -93,8 +93,10 @@ int pycles_device_count(void);
  * passes run (for timing one kernel; a partial call is not a full update).
  * The y and z passes run as one fused kernel when both are selected, the
  * orders are 5 and 5 and the call has momentum and at least one scalar: by
- * default for FP32 storage; PYCLES_ADV_FUSE_YZ asks for it in FP64 as well
- * (same bits as the separate passes; for tests, it is slower there). */
+ * default for FP32 storage and, in FP64, for grids of no more than 256 of its
+ * blocks (64 x 4 columns by a chunk of levels); PYCLES_ADV_FUSE_YZ asks for it
+ * in FP64 on any grid (same bits as the separate passes; for tests, it is slower
+ * on larger ones). */
 #define PYCLES_ADV_TEND_ZERO 1
 #define PYCLES_ADV_PASS_X 2
 #define PYCLES_ADV_PASS_Y 4

@@ -97,9 +97,11 @@ struct PolicyF64 {
     using TC = double;
     using SFlux = double;
     static constexpr bool kBase = false;
-    // the y and z passes stay separate unless asked (PYCLES_ADV_FUSE_YZ, for
-    // tests): the fused kernel's double-buffered FP64 tiles (86 KB of LDS)
-    // leave one block per CU
+    // the y and z passes stay separate unless the grid has no more blocks than
+    // CUs or the caller asks (PYCLES_ADV_FUSE_YZ, for tests): the fused kernel's
+    // double-buffered FP64 tiles (86 KB of LDS) leave one block per CU.  With
+    // one block per CU there is nothing to lose: 64 x 64 x 75 30 us against 19 +
+    // 17, 64^3 23.5 against 12 + 13, and a launch less.
     static constexpr bool kFuseYZ = false;
     static constexpr int kYZWaves = 1;
     // waves per SIMD the z pass is held to (<= 168 VGPRs): its stage-2 form
@@ -1510,7 +1512,7 @@ int launch(const Geo &g, const Prof &pr, const Fields &fl, hipStream_t st) {
     }
     // y and z fused (WENO5 with momentum and scalars), z-chunked like the z pass
     if constexpr (SO == 5 && MO == 5 && MOM && NSC >= 1) {
-        if ((fl.passes & 6) == 6 && (P::kFuseYZ || fl.fuse_yz)) {
+        if ((fl.passes & 6) == 6 && (P::kFuseYZ || fl.fuse_yz || advyz_blocks(g.nx, g.ny, g.nz) <= 256)) {
             // 4 rows per block: 8 rows halve the lower faces' extra work but
             // need more registers than 4 waves per SIMD allow with the RK3
             // stage (spills), and at 3 waves a 512-thread block fits once per CU

@@ -122,6 +122,10 @@ static inline ZSplit advyz_zsplit(int nx, int ny, int nz) {
     const ZSplit z = advz_zsplit(nx, ny, nz);
     return z.len > ADV_YZ_KMAX ? zsplit_ceil(nz, (nz + ADV_YZ_KMAX - 1) / ADV_YZ_KMAX) : z;
 }
+// Its blocks.
+static inline long long advyz_blocks(int nx, int ny, int nz) {
+    return (long long)((nx + 63) / 64) * ((ny + 3) / 4) * advyz_zsplit(nx, ny, nz).nch;
+}
 // The thermodynamics kernels' chunks of the nzg ghosted levels (their LDS
 // holds len + 2 levels, so no chunk is longer than len): up to 4096 blocks.
 // Each chunk evaluates up to two levels of its neighbours, so chunks hold at
