@@ -47,6 +47,9 @@ struct pycles_pressure_plan {
     double *mean, *partial;
     int logx, logy, loggx;
     bool thomas_lds;  // few columns: the z solve with stored pivots, in LDS
+    int planes;       // fewer still: y transforms and z solve of a kx plane in one
+                      // kernel (1; 2: with its pivots staged in LDS)
+    size_t plane_lds;
 };
 
 static int ilog2(long long n) {
@@ -163,7 +166,7 @@ __device__ __forceinline__ void stockham_pass(C2<T> *buf, int S, int b, int t, i
 // sequences in buf, N = 2^logN >= 8, in natural order in and out.
 // tw[m] = exp(-2 pi i m/N), m < N.
 template <typename T, bool INV>
-__device__ void stockham_fft(C2<T> *buf, int S, int b, int t, int N, int logN, const C2<T> *tw, bool act = true) {
+__device__ __forceinline__ void stockham_fft(C2<T> *buf, int S, int b, int t, int N, int logN, const C2<T> *tw, bool act = true) {
     int Ns = 1;
     const int rem = logN % 3;
     if (rem == 1) {
@@ -188,7 +191,9 @@ __device__ void stockham_fft(C2<T> *buf, int S, int b, int t, int N, int logN, c
 // order), then the forward FFT along x of the rows in pairs (row 2b as the
 // real part and row 2b+1 as the imaginary part of one complex sequence),
 // separated into the two half spectra.
-template <typename TS>
+// TR: the spectrum as planes [kx][level][y] (plane_solve_kernel) instead of rows
+// [level][y][kx]; the block's 2S rows are then consecutive.
+template <typename TS, bool TR>
 __global__ __launch_bounds__(512) void div_fftx_kernel(Geo g, const TS *u, const TS *v, const TS *w,
                                                        const double *alpha0, const double *alpha0_half,
                                                        const double *partial, double *mean, double *cfl, TS *div_out,
@@ -286,6 +291,17 @@ __global__ __launch_bounds__(512) void div_fftx_kernel(Geo g, const TS *u, const
     const int b = threadIdx.x & (S - 1), t = threadIdx.x >> logS;
     stockham_fft<TS, false>(buf, S, b, t, g.nx, logx, tw, t < g.nx / 8);
     // X_a[m] = (Z[m] + conj Z[N-m]) / 2, X_b[m] = -i (Z[m] - conj Z[N-m]) / 2
+    if (TR) {
+        for (int q = threadIdx.x; q < nxh * 2 * S; q += blockDim.x) {
+            const int r = q & (2 * S - 1), m = q >> (logS + 1), pb = r >> 1;
+            const C2<TS> z = buf[m * S + pb];
+            const C2<TS> zm = buf[((g.nx - m) & (g.nx - 1)) * S + pb];
+            spec[((long long)m * g.nz + kk) * g.ny + j0 + r] =
+                (r & 1) ? C2<TS>{TS(0.5) * (z.y + zm.y), TS(-0.5) * (z.x - zm.x)}
+                        : C2<TS>{TS(0.5) * (z.x + zm.x), TS(0.5) * (z.y - zm.y)};
+        }
+        return;
+    }
     for (int q = threadIdx.x; q < nxh * S; q += blockDim.x) {
         const int m = q % nxh, pb = q / nxh;
         const C2<TS> z = buf[m * S + pb];
@@ -516,23 +532,86 @@ constexpr int TL_COLS = 16, TL_U = 8;
 template <typename TS> constexpr size_t thomas_lds_bytes(int nz) {
     return (size_t)nz * (TL_COLS * (sizeof(C2<TS>) + sizeof(double) + sizeof(TS)) + sizeof(double));
 }
-// m and c' (rounded to TS, as the forward values are) of column c = ky nxh + kx,
-// [nz][ny nxh]
+// m and c' (rounded to TS, as the forward values are) of column (kx, ky) at
+// level k, at k sk + ky sy + kx sx
 template <typename TS>
 __global__ __launch_bounds__(64) void pivot_kernel(Geo g, const double *kx2, const double *ky2, const double *rho_h,
                                                    const double *dd, const double *a, const double *c, int nxh,
-                                                   double *pm, TS *pc) {
+                                                   long long sk, long long sy, long long sx, double *pm, TS *pc) {
     const long long ncol = (long long)g.ny * nxh;
     const long long col = (long long)blockIdx.x * 64 + threadIdx.x;
     if (col >= ncol) return;
-    const double kk = kx2[col % nxh] + ky2[col / nxh];
+    const int kx = (int)(col % nxh), ky = (int)(col / nxh);
+    const double kk = kx2[kx] + ky2[ky];
+    const long long o = ky * sy + kx * sx;
     double sc = 0.0;
     for (int k = 0; k < g.nz; ++k) {
         const double b = rho_h[k] * kk - dd[k];
         const double m = k == 0 ? rcp64(b) : rcp64(b - a[k] * sc);
         sc = c[k] * m;
-        pm[k * ncol + col] = m;
-        pc[k * ncol + col] = (TS)sc;
+        pm[k * sk + o] = m;
+        pc[k * sk + o] = (TS)sc;
+    }
+}
+// Both sweeps of one part (real or imaginary) of one column from the stored
+// pivots: x[k xs] in LDS holds the right-hand side and becomes the solution,
+// m[k ms] and c[k ms] (LDS or global) are the pivots' arrays, la the lower
+// diagonal.  A batch of TL_U levels is read while the one before is worked on.
+template <typename TS>
+__device__ __forceinline__ void column_sweeps(TS *x, int xs, const double *m, const TS *c, long long ms, const double *la,
+                                              int nz) {
+    double xr = 0.0;
+    TS q[2][TL_U];
+    double pm[2][TL_U], pa[2][TL_U];
+    auto fetch = [&](int b, int k0) {
+#pragma unroll
+        for (int u = 0; u < TL_U; ++u) {
+            const int k = min(k0 + u, nz - 1);
+            q[b][u] = x[k * xs];
+            pm[b][u] = m[k * ms];
+            pa[b][u] = la[k];
+        }
+    };
+    auto fwd = [&](int b, int k0) {
+#pragma unroll
+        for (int u = 0; u < TL_U; ++u)
+            if (k0 + u < nz) {
+                xr = k0 + u == 0 ? (double)q[b][u] * pm[b][u] : ((double)q[b][u] - pa[b][u] * xr) * pm[b][u];
+                x[(k0 + u) * xs] = (TS)xr;
+            }
+    };
+    fetch(0, 0);
+    for (int k0 = 0; k0 < nz; k0 += 2 * TL_U) {
+        fetch(1, k0 + TL_U);
+        fwd(0, k0);
+        fetch(0, k0 + 2 * TL_U);
+        fwd(1, k0 + TL_U);
+    }
+    // back substitution from the level below the top, whose solution is its
+    // forward value, carried unrounded
+    TS f[2][TL_U];
+    auto bfetch = [&](int b, int k0) {
+#pragma unroll
+        for (int u = 0; u < TL_U; ++u) {
+            const int k = max(k0 - u, 0);
+            q[b][u] = x[k * xs];
+            f[b][u] = c[k * ms];
+        }
+    };
+    auto bwd = [&](int b, int k0) {
+#pragma unroll
+        for (int u = 0; u < TL_U; ++u)
+            if (k0 - u >= 0) {
+                xr = (double)q[b][u] - (double)f[b][u] * xr;
+                x[(k0 - u) * xs] = (TS)xr;
+            }
+    };
+    bfetch(0, nz - 2);
+    for (int k0 = nz - 2; k0 >= 0; k0 -= 2 * TL_U) {
+        bfetch(1, k0 - TL_U);
+        bwd(0, k0);
+        bfetch(0, k0 - 2 * TL_U);
+        bwd(1, k0 - TL_U);
     }
 }
 template <typename TS>
@@ -575,63 +654,8 @@ __global__ __launch_bounds__(256) void thomas_lds_kernel(Geo g, C2<TS> *spec, co
     }
     __syncthreads();
     if (threadIdx.x < 2 * TL_COLS) {
-        TS *x = reinterpret_cast<TS *>(z) + 2 * cl + threadIdx.x / TL_COLS;  // this lane's part, level stride 2 TL_COLS
-        const double *m = lm + cl;
-        const TS *f = lc + cl;
-        double xr = 0.0;
-        // forward, a batch of TL_U levels read while the one before is worked on
-        TS q[2][TL_U];
-        double pm_[2][TL_U], pa[2][TL_U];
-        auto fetch = [&](int b, int k0) {
-#pragma unroll
-            for (int u = 0; u < TL_U; ++u) {
-                const int k = min(k0 + u, nz - 1);
-                q[b][u] = x[k * 2 * TL_COLS];
-                pm_[b][u] = m[k * TL_COLS];
-                pa[b][u] = la[k];
-            }
-        };
-        auto fwd = [&](int b, int k0) {
-#pragma unroll
-            for (int u = 0; u < TL_U; ++u)
-                if (k0 + u < nz) {
-                    xr = k0 + u == 0 ? (double)q[b][u] * pm_[b][u] : ((double)q[b][u] - pa[b][u] * xr) * pm_[b][u];
-                    x[(k0 + u) * 2 * TL_COLS] = (TS)xr;
-                }
-        };
-        fetch(0, 0);
-        for (int k0 = 0; k0 < nz; k0 += 2 * TL_U) {
-            fetch(1, k0 + TL_U);
-            fwd(0, k0);
-            fetch(0, k0 + 2 * TL_U);
-            fwd(1, k0 + TL_U);
-        }
-        // back substitution from the level below the top, whose solution is
-        // its forward value, carried unrounded
-        TS fq[2][TL_U];
-        auto bfetch = [&](int b, int k0) {
-#pragma unroll
-            for (int u = 0; u < TL_U; ++u) {
-                const int k = max(k0 - u, 0);
-                q[b][u] = x[k * 2 * TL_COLS];
-                fq[b][u] = f[k * TL_COLS];
-            }
-        };
-        auto bwd = [&](int b, int k0) {
-#pragma unroll
-            for (int u = 0; u < TL_U; ++u)
-                if (k0 - u >= 0) {
-                    xr = (double)q[b][u] - (double)fq[b][u] * xr;
-                    x[(k0 - u) * 2 * TL_COLS] = (TS)xr;
-                }
-        };
-        bfetch(0, nz - 2);
-        for (int k0 = nz - 2; k0 >= 0; k0 -= 2 * TL_U) {
-            bfetch(1, k0 - TL_U);
-            bwd(0, k0);
-            bfetch(0, k0 - 2 * TL_U);
-            bwd(1, k0 - TL_U);
-        }
+        column_sweeps<TS>(reinterpret_cast<TS *>(z) + 2 * cl + threadIdx.x / TL_COLS, 2 * TL_COLS, lm + cl, lc + cl, TL_COLS,
+                          la, nz);
     }
     __syncthreads();
     // the (0,0) mode is set to zero
@@ -641,11 +665,93 @@ __global__ __launch_bounds__(256) void thomas_lds_kernel(Geo g, C2<TS> *spec, co
             sp[(long long)k * plane] = zero ? C2<TS>{TS(0), TS(0)} : z[k * TL_COLS + cl];
 }
 
+// The transform along y, the z solve and the inverse transform of one
+// wavenumber kx in one kernel, where a plane of ny x nz complex values fits in
+// LDS and the nxh planes' blocks are all resident at once: three kernels of
+// little work each (two transforms and the solve, 22 us at 64^3 FP64) become one
+// and the spectrum is read and written once instead of three times.  The
+// spectrum is laid out as planes [kx][level][y].  In LDS level b of row y is
+// element y S + b, S = nz made odd, so that accesses along either index spread
+// over the banks.  The transforms run over as many levels at a time as the
+// block has threads (ny / 8 each), the sweeps on one lane per column and part.
+// The same bits as the separate kernels.  64^3 FP64 22.5 -> 17.7 us, 256 x 64 x 75
+// FP32 29 -> 19, and two launches less.
+// ST: the plane's pivots are staged in LDS too, loaded with the spectrum (read
+// from global memory the sweeps wait for them).
+template <typename TS, bool ST> size_t plane_lds_bytes(int ny, int nz) {
+    return sizeof(C2<TS>) * (size_t)ny * (nz | 1) + sizeof(double) * (size_t)nz +
+           (ST ? (sizeof(double) + sizeof(TS)) * (size_t)ny * nz : 0);
+}
+template <typename TS, bool ST>
+__global__ __launch_bounds__(1024) void plane_solve_kernel(Geo g, C2<TS> *spec, const double *pm, const TS *pc,
+                                                           const double *a, const C2<TS> *tw, int logy) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    const int ny = g.ny, nz = g.nz, S = nz | 1, B = blockDim.x, tid = threadIdx.x;
+    C2<TS> *buf = reinterpret_cast<C2<TS> *>(smem_raw);
+    double *la = reinterpret_cast<double *>(buf + (size_t)ny * S);
+    double *lm = la + nz;                                        // ST: [nz][ny]
+    TS *lc = reinterpret_cast<TS *>(lm + (ST ? (size_t)nz * ny : 0));
+    const long long plane = (long long)blockIdx.x * nz * ny;
+    C2<TS> *sp = spec + plane;
+    for (int t = tid; t < nz; t += B) la[t] = a[t];
+    const int n = ny * nz;
+    for (int q0 = tid; q0 < n; q0 += 4 * B) {
+        C2<TS> z[4];
+        double m[4];
+        TS f[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int q = min(q0 + u * B, n - 1);
+            z[u] = sp[q];
+            if (ST) {
+                m[u] = pm[plane + q];
+                f[u] = pc[plane + q];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int q = q0 + u * B;
+            if (q < n) {
+                buf[(q & (ny - 1)) * S + (q >> logy)] = z[u];
+                if (ST) {
+                    lm[q] = m[u];
+                    lc[q] = f[u];
+                }
+            }
+        }
+    }
+    __syncthreads();
+    const int n8 = ny >> 3;
+    const int per = min(B / n8, nz);  // levels transformed at a time
+    const int b = tid % per, t = tid / per;
+    for (int l0 = 0; l0 < nz; l0 += per)
+        stockham_fft<TS, false>(buf + l0, S, b, t, ny, logy, tw, t < n8 && l0 + b < nz);
+    for (int c = tid; c < 2 * ny; c += B) {
+        const int ky = c & (ny - 1);
+        column_sweeps<TS>(reinterpret_cast<TS *>(buf + (size_t)ky * S) + (c >> logy), 2, (ST ? lm : pm + plane) + ky,
+                          (ST ? lc : pc + plane) + ky, ny, la, nz);
+    }
+    __syncthreads();
+    if (blockIdx.x == 0) {  // the (0,0) mode is set to zero
+        for (int k = tid; k < nz; k += B) buf[k] = C2<TS>{TS(0), TS(0)};
+        __syncthreads();
+    }
+    for (int l0 = 0; l0 < nz; l0 += per)
+        stockham_fft<TS, true>(buf + l0, S, b, t, ny, logy, tw, t < n8 && l0 + b < nz);
+    const TS sc = TS(1.0 / (double)ny);
+    for (int q = tid; q < n; q += B) {
+        C2<TS> z = buf[(q & (ny - 1)) * S + (q >> logy)];
+        z.x *= sc;
+        z.y *= sc;
+        sp[q] = z;
+    }
+}
+
 // Inverse x transform of 2S rows in pairs: Z[m] = X_a[m] + i X_b[m] with the
 // Hermitian extension X[N-m] = conj X[m], one inverse FFT, real part -> row
 // 2b and imaginary part -> row 2b+1, times 1/nx, written to p at level k'+gw
 // together with the mirrored z ghost level (sym, as communicate_variable does).
-template <typename TS>
+template <typename TS, bool TR>
 __global__ __launch_bounds__(512) void ifftx_kernel(Geo g, const C2<TS> *spec, TS *p, const C2<TS> *tw, int logx,
                                                     int nxh, int nxp, int logS) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -663,20 +769,26 @@ __global__ __launch_bounds__(512) void ifftx_kernel(Geo g, const C2<TS> *spec, T
         for (int u = 0; u < 4; ++u) {
             const int q = q0 + u * B;
             if (q < nq) {
-                const int m = q & (g.nx - 1);
-                const int pb = q >> logx;
-                const C2<TS> *ra = spec + ((long long)kk * g.ny + j0 + 2 * pb) * nxp;
+                const int m = TR ? q >> logS : q & (g.nx - 1);
+                const int pb = TR ? q & (S - 1) : q >> logx;
                 const int mm = m < nxh ? m : g.nx - m;
-                xa[u] = ra[mm];
-                xb[u] = ra[nxp + mm];
+                if (TR) {  // rows 2 pb and 2 pb + 1 of wavenumber mm are neighbours
+                    const C2<TS> *ra = spec + ((long long)mm * g.nz + kk) * g.ny + j0 + 2 * pb;
+                    xa[u] = ra[0];
+                    xb[u] = ra[1];
+                } else {
+                    const C2<TS> *ra = spec + ((long long)kk * g.ny + j0 + 2 * pb) * nxp;
+                    xa[u] = ra[mm];
+                    xb[u] = ra[nxp + mm];
+                }
             }
         }
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const int q = q0 + u * B;
             if (q < nq) {
-                const int m = q & (g.nx - 1);
-                const int pb = q >> logx;
+                const int m = TR ? q >> logS : q & (g.nx - 1);
+                const int pb = TR ? q & (S - 1) : q >> logx;
                 if (m >= nxh) {  // Hermitian extension X[N-m] = conj X[m]
                     xa[u].y = -xa[u].y;
                     xb[u].y = -xb[u].y;
@@ -910,7 +1022,26 @@ extern "C" int pycles_pressure_plan_create(const pycles_dims *dims, const double
             if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess)
                 P->thomas_lds = false;
         }
-        if (P->thomas_lds) {
+        // the plane form where its blocks are all resident at once and either
+        // half the CUs have one or a plane is little work for the others to
+        // wait for: 256 x 256 x 60 FP32 174 -> 162 us a projection, 64 x 64 x 64
+        // FP64 gains 10 us, 64 x 128 x 70 (33 blocks of 8960 values) would lose 20;
+        // with staged pivots, or else without
+        const bool few = P->nxh >= 128 || (long long)g.ny * nz <= 5120;
+        for (int stg = 1; few && stg >= 0 && !P->planes; --stg) {
+            const size_t pl = precision == PYCLES_F64
+                                  ? (stg ? plane_lds_bytes<double, true>(g.ny, nz) : plane_lds_bytes<double, false>(g.ny, nz))
+                                  : (stg ? plane_lds_bytes<float, true>(g.ny, nz) : plane_lds_bytes<float, false>(g.ny, nz));
+            if (pl > 160 * 1024 || P->nxh > 256 * (int)(160 * 1024 / pl)) continue;
+            P->planes = 1 + stg;
+            P->plane_lds = pl;
+            const void *fn = precision == PYCLES_F64
+                                 ? (stg ? (const void *)plane_solve_kernel<double, true> : (const void *)plane_solve_kernel<double, false>)
+                                 : (stg ? (const void *)plane_solve_kernel<float, true> : (const void *)plane_solve_kernel<float, false>);
+            if (pl > 64 * 1024 && hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess)
+                P->planes = 0;
+        }
+        if (P->planes || P->thomas_lds) {
             ALLOC(P->pm, sizeof(double) * (size_t)g.nz * g.ny * P->nxh);
             ALLOC(P->pc, es * (size_t)g.nz * g.ny * P->nxh);
         } else {
@@ -951,14 +1082,17 @@ extern "C" int pycles_pressure_plan_create(const pycles_dims *dims, const double
         pycles_pressure_plan_destroy(P);
         return PYCLES_ERR_HIP;
     }
-    if (P->thomas_lds) {
+    if (P->planes || P->thomas_lds) {
         const dim3 grid((unsigned)(((long long)g.ny * P->nxh + 63) / 64));
+        // planes: [kx][level][ky]; otherwise [level][ky][kx]
+        const long long sk = P->planes ? g.ny : (long long)g.ny * P->nxh, sy = P->planes ? 1 : P->nxh,
+                        sx = P->planes ? (long long)g.nz * g.ny : 1;
         if (precision == PYCLES_F64)
             hipLaunchKernelGGL(pivot_kernel<double>, grid, dim3(64), 0, 0, g, P->kx2, P->ky2, P->rho_h, P->dd, P->a, P->c,
-                               P->nxh, P->pm, (double *)P->pc);
+                               P->nxh, sk, sy, sx, P->pm, (double *)P->pc);
         else
             hipLaunchKernelGGL(pivot_kernel<float>, grid, dim3(64), 0, 0, g, P->kx2, P->ky2, P->rho_h, P->dd, P->a, P->c,
-                               P->nxh, P->pm, (float *)P->pc);
+                               P->nxh, sk, sy, sx, P->pm, (float *)P->pc);
         e = hipGetLastError();
         if (e == hipSuccess) e = hipStreamSynchronize(0);  // any stream may use the plan
         if (e != hipSuccess) {
@@ -1000,31 +1134,54 @@ static int run_pressure(pycles_pressure_plan *P, const pycles_ref *ref, void *u,
     const int bx = S * g.nx / 8;
     const long long waves = (long long)(g.ny / (2 * S)) * g.nz * ((bx + 63) / 64);
     const int dbx = waves < 4096 && bx >= 32 && bx <= 128 ? 4 * bx : bx;
-    hipLaunchKernelGGL(div_fftx_kernel<TS>, dim3(g.ny / (2 * S), g.nz), dim3(dbx), rowsmem, st, g, (const TS *)u,
-                       (const TS *)v, (const TS *)w, ref->alpha0, ref->alpha0_half, P->partial, P->mean, cfl_out,
-                       (TS *)div, (C2<TS> *)P->spec, (const C2<TS> *)P->twx, P->logx, P->nxh, P->nxp, logS);
+#define DIV_FFTX(TR_)                                                                                          \
+    hipLaunchKernelGGL((div_fftx_kernel<TS, TR_>), dim3(g.ny / (2 * S), g.nz), dim3(dbx), rowsmem, st, g,       \
+                       (const TS *)u, (const TS *)v, (const TS *)w, ref->alpha0, ref->alpha0_half, P->partial,  \
+                       P->mean, cfl_out, (TS *)div, (C2<TS> *)P->spec, (const C2<TS> *)P->twx, P->logx, P->nxh, \
+                       P->nxp, logS)
+    if (P->planes) DIV_FFTX(true);
+    else DIV_FFTX(false);
+#undef DIV_FFTX
     PYCLES_CHECK_LAUNCH();
-    const size_t ysmem = sizeof(C2<TS>) * (size_t)g.ny * P->gx;
-    const dim3 ygrid((P->nxh + P->gx - 1) / P->gx, g.nz);
-    const int by = P->gx * g.ny / 8;
-    hipLaunchKernelGGL(ffty_kernel<TS>, ygrid, dim3(by), ysmem, st, g, (C2<TS> *)P->spec,
-                       (const C2<TS> *)P->twy, P->logy, P->nxh, P->nxp, P->gx, P->loggx, 0);
-    PYCLES_CHECK_LAUNCH();
-    const long long ncol = (long long)g.ny * P->nxp;
-    if (P->thomas_lds)
-        hipLaunchKernelGGL(thomas_lds_kernel<TS>, dim3((unsigned)(((long long)g.ny * P->nxh + TL_COLS - 1) / TL_COLS)),
-                           dim3(256), thomas_lds_bytes<TS>(g.nz), st, g, (C2<TS> *)P->spec, P->pm, (const TS *)P->pc,
-                           P->a, P->nxh, P->nxp);
-    else
-        hipLaunchKernelGGL((thomas_kernel<TS, thomas_seg<TS>()>), dim3((unsigned)((ncol + 255) / 256)), dim3(256),
-                           4 * sizeof(double) * (size_t)g.nz, st, g, (C2<TS> *)P->spec, P->ck, P->kx2, P->ky2,
-                           P->rho_h, P->dd, P->a, P->c, P->nxh, P->nxp);
-    PYCLES_CHECK_LAUNCH();
-    hipLaunchKernelGGL(ffty_kernel<TS>, ygrid, dim3(by), ysmem, st, g, (C2<TS> *)P->spec,
-                       (const C2<TS> *)P->twy, P->logy, P->nxh, P->nxp, P->gx, P->loggx, 1);
-    PYCLES_CHECK_LAUNCH();
-    hipLaunchKernelGGL(ifftx_kernel<TS>, dim3(g.ny / (2 * S), g.nz), dim3(bx), rowsmem, st, g,
-                       (const C2<TS> *)P->spec, (TS *)p, (const C2<TS> *)P->twx, P->logx, P->nxh, P->nxp, logS);
+    if (P->planes) {
+        // threads for all levels' transforms, or for the sweeps, up to 1024
+        int pb = g.nz * (g.ny / 8);
+        if (pb < 2 * g.ny) pb = 2 * g.ny;
+        pb = pb > 1024 ? 1024 : (pb + 63) / 64 * 64;
+        if (P->planes == 2)
+            hipLaunchKernelGGL((plane_solve_kernel<TS, true>), dim3(P->nxh), dim3(pb), P->plane_lds, st, g,
+                               (C2<TS> *)P->spec, P->pm, (const TS *)P->pc, P->a, (const C2<TS> *)P->twy, P->logy);
+        else
+            hipLaunchKernelGGL((plane_solve_kernel<TS, false>), dim3(P->nxh), dim3(pb), P->plane_lds, st, g,
+                               (C2<TS> *)P->spec, P->pm, (const TS *)P->pc, P->a, (const C2<TS> *)P->twy, P->logy);
+        PYCLES_CHECK_LAUNCH();
+    } else {
+        const size_t ysmem = sizeof(C2<TS>) * (size_t)g.ny * P->gx;
+        const dim3 ygrid((P->nxh + P->gx - 1) / P->gx, g.nz);
+        const int by = P->gx * g.ny / 8;
+        hipLaunchKernelGGL(ffty_kernel<TS>, ygrid, dim3(by), ysmem, st, g, (C2<TS> *)P->spec,
+                           (const C2<TS> *)P->twy, P->logy, P->nxh, P->nxp, P->gx, P->loggx, 0);
+        PYCLES_CHECK_LAUNCH();
+        const long long ncol = (long long)g.ny * P->nxp;
+        if (P->thomas_lds)
+            hipLaunchKernelGGL(thomas_lds_kernel<TS>, dim3((unsigned)(((long long)g.ny * P->nxh + TL_COLS - 1) / TL_COLS)),
+                               dim3(256), thomas_lds_bytes<TS>(g.nz), st, g, (C2<TS> *)P->spec, P->pm, (const TS *)P->pc,
+                               P->a, P->nxh, P->nxp);
+        else
+            hipLaunchKernelGGL((thomas_kernel<TS, thomas_seg<TS>()>), dim3((unsigned)((ncol + 255) / 256)), dim3(256),
+                               4 * sizeof(double) * (size_t)g.nz, st, g, (C2<TS> *)P->spec, P->ck, P->kx2, P->ky2,
+                               P->rho_h, P->dd, P->a, P->c, P->nxh, P->nxp);
+        PYCLES_CHECK_LAUNCH();
+        hipLaunchKernelGGL(ffty_kernel<TS>, ygrid, dim3(by), ysmem, st, g, (C2<TS> *)P->spec,
+                           (const C2<TS> *)P->twy, P->logy, P->nxh, P->nxp, P->gx, P->loggx, 1);
+        PYCLES_CHECK_LAUNCH();
+    }
+#define IFFTX(TR_)                                                                                             \
+    hipLaunchKernelGGL((ifftx_kernel<TS, TR_>), dim3(g.ny / (2 * S), g.nz), dim3(bx), rowsmem, st, g,           \
+                       (const C2<TS> *)P->spec, (TS *)p, (const C2<TS> *)P->twx, P->logx, P->nxh, P->nxp, logS)
+    if (P->planes) IFFTX(true);
+    else IFFTX(false);
+#undef IFFTX
     PYCLES_CHECK_LAUNCH();
     const ZSplit zs = correct_zsplit(g.plane, g.nz, g.gw);
     constexpr int V = 16 / sizeof(TS);

@@ -308,10 +308,12 @@ def test_dry_thermo_tiles(n, gw, precision):
 
 @pytest.mark.parametrize("n,gw,shift", [((8, 8, 5), 5, 0), ((16, 8, 9), 3, 1), ((8, 64, 2), 2, 0), ((64, 64, 64), 3, 0),
                                         ((32, 16, 104), 3, 1), ((16, 8, 315), 3, 0), ((16, 8, 316), 3, 0),
-                                        ((256, 128, 12), 3, 0), ((512, 256, 3), 3, 1)])
+                                        ((256, 128, 12), 3, 0), ((512, 256, 3), 3, 1), ((64, 128, 40), 3, 0), ((64, 128, 41), 3, 0),
+                                        ((256, 64, 75), 3, 0), ((256, 64, 160), 3, 0), ((8, 1024, 5), 3, 0)])
 def test_projection_forms(n, gw, shift):
-    """The projection in the forms its size rules choose (few columns with
-    stored pivots in LDS, up to 315 FP64 levels; blocks of less than half a
+    """The projection in the forms its size rules choose (kx planes in one
+    kernel, with and without staged pivots; few columns with stored pivots in
+    LDS, up to 315 FP64 levels; the general solve; blocks of less than half a
     wavefront; few and many sequences per block) and off a 16-byte boundary (shift), FP64 against the
     oracle: 1e-12 of each field's maximum, as test_pressure_parity.  The CFL
     maximum is exact for the velocities that come back."""
