@@ -98,25 +98,25 @@ __global__ __launch_bounds__(256) void thermo_sa_f64_kernel(Geo g, SAArgs a) {
             double thr = 0.0;
             if (k >= 1 && k < g.nzg - 1) thr = T * (1.0 - qt + PC_EPS_VI * qv) / ex;
             if (own) {
-                To[o] = T;
-                qvo[o] = qv;
-                qlo[o] = ql;
-                alo[o] = al;
-                if (bo && k < g.nzg - 1) bo[o] = b;
-                if (thro && k >= 1 && k < g.nzg - 1) thro[o] = thr;
+                put_nt(To + o, T);
+                put_nt(qvo + o, qv);
+                put_nt(qlo + o, ql);
+                put_nt(alo + o, al);
+                if (bo && k < g.nzg - 1) put_nt(bo + o, b);
+                if (thro && k >= 1 && k < g.nzg - 1) put_nt(thro + o, thr);
                 if (thlo) {
                     // exp(-L*0/(T cpd)) is exactly 1 for unsaturated cells
-                    if (ql == 0.0 && qi == 0.0) thlo[o] = T / ex * 1.0;
+                    if (ql == 0.0 && qi == 0.0) put_nt(thlo + o, T / ex * 1.0);
                     else {
                         const double L = thermo::latent_heat_variable(T);
-                        thlo[o] = T / ex * exp(-L * (ql / (1.0 - qt) + qi / (1.0 - qt)) / (T * PC_CPD));
+                        put_nt(thlo + o, T / ex * exp(-L * (ql / (1.0 - qt) + qi / (1.0 - qt)) / (T * PC_CPD)));
                     }
                 }
             }
             // w tendency at k-1 for k-1 in [1, nzg-3): wt + interp_2(b[k-1], b[k])
             if (own_m && k >= 2 && k - 1 < g.nzg - 3) {
                 const double w0 = WTO ? 0.0 : wt[o - g.plane];
-                wt[o - g.plane] = w0 + 0.5 * (bprev + b);
+                put_nt(wt + o - g.plane, w0 + 0.5 * (bprev + b));
             }
             bprev = b;
             Tw[0] = Tw[1]; Tw[1] = Tw[2]; Tw[2] = T;
@@ -125,7 +125,7 @@ __global__ __launch_bounds__(256) void thermo_sa_f64_kernel(Geo g, SAArgs a) {
             thw[0] = thw[1]; thw[1] = thw[2]; thw[2] = thr;
             const int m = k - 1;
             if (bvfo && own_m && m >= 2 && m < g.nzg - 2)
-                bvfo[o - g.plane] = thermo::bvf_sa<thermo::DivFast>(lt, p0l[l - 1], Tw, qtw, qvw, thw, dzi);
+                put_nt(bvfo + o - g.plane, thermo::bvf_sa<thermo::DivFast>(lt, p0l[l - 1], Tw, qtw, qvw, thw, dzi));
         }
     }
     flush_counters(cnt, ctr, a.counters, tid);

@@ -150,24 +150,24 @@ __global__ __launch_bounds__(256, MLP ? 4 : 5) void thermo_sa_f32_kernel(Geo g, 
         qvw[0] = qvw[1]; qvw[1] = qvw[2]; qvw[2] = qv;
         thw[0] = thw[1]; thw[1] = thw[2]; thw[2] = thr;
         if (own) {
-            To[o] = T;
-            qvo[o] = qv;
-            qlo[o] = ql;
-            alo[o] = al;
-            if (bo && k < g.nzg - 1) bo[o] = b;
-            if (thro && k >= 1 && k < g.nzg - 1) thro[o] = thr;
+            put_nt(To + o, T);
+            put_nt(qvo + o, qv);
+            put_nt(qlo + o, ql);
+            put_nt(alo + o, al);
+            if (bo && k < g.nzg - 1) put_nt(bo + o, b);
+            if (thro && k >= 1 && k < g.nzg - 1) put_nt(thro + o, thr);
             if (thlo) {
-                if (ql == 0.0f) thlo[o] = T * iex;
+                if (ql == 0.0f) put_nt(thlo + o, T * iex);
                 else {
                     const float L = thermo32::latent_heat(T);
-                    thlo[o] = T * iex *
-                              thermo32::fexp(-L * thermo32::fdiv(thermo32::fdiv(ql, 1.0f - qt), T * (float)PC_CPD));
+                    put_nt(thlo + o, T * iex *
+                                         thermo32::fexp(-L * thermo32::fdiv(thermo32::fdiv(ql, 1.0f - qt), T * (float)PC_CPD)));
                 }
             }
         }
         if (own_m && k >= 2 && k - 1 < g.nzg - 3) {
             const float w0 = WTO ? 0.0f : wt[o - g.plane];
-            wt[o - g.plane] = w0 + 0.5f * (bprev + b);
+            put_nt(wt + o - g.plane, w0 + 0.5f * (bprev + b));
         }
         bprev = b;
         const int m = k - 1;
@@ -195,7 +195,7 @@ __global__ __launch_bounds__(256, MLP ? 4 : 5) void thermo_sa_f32_kernel(Geo g, 
             } else {
                 bv = (float)PC_G * thermo32::frcp(thw[1]) * 0.5f * (thw[2] - thw[0]) * dzi;
             }
-            bvfo[o - g.plane] = bv;
+            put_nt(bvfo + o - g.plane, bv);
         }
     }
     const unsigned long long ctr64[4] = {ctr[0], ctr[1], ctr[2], ctr[3]};
