@@ -448,3 +448,64 @@ def test_advection_x_forms_bitwise(n, orders, moist, shift):
             got = slot(len(names) + q).cpu().numpy().reshape(nzg, ny, nx)[gw:-gw]
             want = np.asarray(sim.pt(k))[gw:-gw, gw:-gw, gw:-gw].transpose(2, 1, 0)
             assert np.array_equal(got, want), (k, zero, np.abs(got - want).max())
+
+
+@pytest.mark.parametrize("n,orders", [((70, 9, 13), (5, 5)), ((64, 12, 70), (5, 5)), ((33, 11, 9), (7, 7)), ((65, 10, 150), (9, 5)),
+                                      ((24, 13, 21), (9, 9))])
+@pytest.mark.parametrize("moist", [True, False])
+def test_fp32_advection_forms(n, orders, moist):
+    """FP32 tendencies against the FP64 oracle on the same values, at every
+    order, over partial tiles and several z chunks, with level profiles that
+    change by more than the deviations from one level to the next (moist) and
+    without profiles (dry).  Bound: with D the largest offset in a window, a
+    face's reconstruction is within 400 eps D (weights and candidates: about
+    30 operations each on terms of up to 6 D, and the rounded profile
+    differences), twice per direction; the parts of a tendency round to eps
+    of their size at each of the passes' additions."""
+    import torch
+    from oracle import oracle as O
+    from pycles_amd import _capi
+    from pycles_amd import _device as D
+    nx, ny, nz = n
+    gw = (max(orders) + 1) // 2
+    nzg = nz + 2 * gw
+    dx = (50.0, 60.0, 20.0)
+    rng = np.random.default_rng(nx + ny + nz)
+    alpha = 0.8 + 0.3 * np.arange(nzg) / nzg
+    half = alpha - 0.004
+    prof = {"rho0": 1.0 / alpha, "rho0_half": 1.0 / half, "alpha0": alpha, "alpha0_half": half, "p0": alpha, "p0_half": alpha}
+    oref = O.Ref(prof["p0"], prof["p0_half"], alpha, half, prof["rho0"], prof["rho0_half"])
+    dp = {k: _dev(v) for k, v in prof.items()}
+    ref = _capi.Ref(*[dp[k].data_ptr() for k in ("rho0", "rho0_half", "alpha0", "alpha0_half", "p0", "p0_half")])
+    names = ["u", "v", "w", "s"] + (["qt"] if moist else [])
+    f = {k: rng.standard_normal((nzg, ny, nx)).astype(np.float32) for k in names}
+    base = {k: np.cumsum(rng.uniform(-3.0, 5.0, nzg)) for k in names[3:]} if moist else {}
+    lt = O.Lookup(np.linspace(100.0, 380.0, 16), np.linspace(1.0, 2.0, 16)) if moist else None
+    sim = O.OracleSimulation(O.make_dims(nx, ny, nz, gw, *dx), oref, moist, lt, scalar_order=orders[0],
+                             momentum_order=orders[1])
+    dev, tend = {}, {}
+    for k in names:
+        full = f[k].astype(np.float64) + (base[k][:, None, None] if k in base else 0.0)
+        sim.pv(k)[...] = np.pad(full.transpose(2, 1, 0), ((gw, gw), (gw, gw), (0, 0)), mode="wrap")
+        sim.pt(k)[...] = 0.0
+        dev[k], tend[k] = _dev(f[k]), torch.zeros((nzg, ny, nx), dtype=torch.float32, device="cuda")
+    sim.scalar_advection_update()
+    sim.momentum_advection_update()
+    bd = {k: _dev(v) for k, v in base.items()}
+    sb = _capi.ScalarBase(*[bd[k].data_ptr() for k in names[3:]]) if moist else None
+    _capi.advection(_dims(n, gw, dx), ref, [dev[k].data_ptr() for k in names[:3]], [tend[k].data_ptr() for k in names[:3]],
+                    [dev[k].data_ptr() for k in names[3:]], [tend[k].data_ptr() for k in names[3:]], sb, *orders, D.F32,
+                    D.stream(), 0)
+    eps = np.finfo(np.float32).eps
+    umax = 1.5 * max(np.abs(f[k]).max() for k in names[:3])  # a centred value is at most (4/3) max
+    for k in names:
+        amp = np.abs(f[k]).max()
+        b = base.get(k, np.zeros(nzg))
+        jump = max(np.abs(b[m:] - b[:-m]).max() for m in range(1, 6))
+        scale = 2.0 * umax * 1.4 * sum(1.0 / d for d in dx)  # two faces of each direction, alpha rho
+        tol = scale * (400 * eps * (2 * amp + jump) + 8 * eps * (amp + np.abs(b).max()))
+        got = tend[k].cpu().numpy()[gw:-gw].astype(np.float64)
+        want = np.asarray(sim.pt(k))[gw:-gw, gw:-gw, gw:-gw].transpose(2, 1, 0)
+        err = np.abs(got - want).max()
+        print(k, "error / bound", err / tol, flush=True)
+        assert err <= tol, (k, err, tol)
