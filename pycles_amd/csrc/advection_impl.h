@@ -112,7 +112,7 @@ struct PolicyF64 {
     static constexpr int kXThreads = 512;
     static constexpr int kXWaves5 = 4;     // waves per SIMD it is held to at WENO5 (128 VGPRs)
     template <int O, bool BV>
-    static __device__ __forceinline__ SFlux scal_flux(const TC *win, const double *, TC U, double rho) {
+    static __device__ __forceinline__ SFlux scal_flux(const TC *win, const float *, const double *, TC U, double rho) {
         return upwind_flux<O, double>(win, U, rho);
     }
     template <int O>
@@ -136,6 +136,36 @@ struct PolicyF64 {
 };
 
 // -------------------------------------------------------------------------
+// z windows of FP32 scalars: what the level profile adds to the offsets from
+// the upwind centre depends on the face and the wind's sign only.  A block
+// forms it once for the faces of its chunk, in FP64 and rounded, in LDS: per
+// face one row for each upwind side (U >= 0, U < 0) of the 2R - 2 differences
+// of the profile to its value at the centre, in window order without the
+// centre, padded to whole 16-byte reads; and the profile itself.  Forming them
+// in every cell took, per window entry, a select, a subtraction and a
+// conversion of 64 bits; the passes are bound by instruction issue (fused y-z
+// pass at 512 x 512 x 256 1.69 -> 1.55 ms, WENO9/5 z pass at 1024 x 1024 x 192
+// 3.54 -> 2.86).
+__host__ __device__ constexpr int base_nd(int R) { return R == 3 ? 4 : 8; }
+// Faces c0 .. c0 + n - 1.
+template <int R, int NSC, int NT>
+__device__ __forceinline__ void base_rows(const Fields &fl, int c0, int n, int ktop, int tid, int nthr,
+                                          float (&dif)[NSC][NT][2][base_nd(R)]) {
+    constexpr int ND = base_nd(R);
+    for (int e = tid; e < NSC * n * 2 * ND; e += nthr) {
+        const int m = e % ND, side = e / ND % 2, f = e / (2 * ND) % n, sc = e / (2 * ND) / n;
+        const double *p = sc == 0 ? fl.base[0] : fl.base[1];
+        float d = 0.0f;
+        if (p && m < 2 * R - 2) {
+            const int c = c0 + f, w = m < R - 1 ? m : m + 1;  // window slot
+            const int lev = c - (R - 1) + (side ? 2 * R - 1 - w : w);
+            d = (float)(p[min(max(lev, 0), ktop)] - p[min(c + side, ktop)]);
+        }
+        dif[sc][f][side][m] = d;
+    }
+}
+
+// -------------------------------------------------------------------------
 // FP32 policy.  Scalars are stored as deviations phi' = phi - base(k) from an
 // FP64 level profile.  The reconstruction is evaluated on offsets from the
 // upwind centre cell, d_m = phi_m - phi_ctr (WENO is invariant to adding a
@@ -144,8 +174,9 @@ struct PolicyF64 {
 // pair: the small part rho*U*(phi'_ctr + R(d)) in FP32 and the base part
 // rho*U*base_ctr in FP64, and the base part's flux difference is formed in
 // FP64 before the tendency is rounded to FP32 (compensated flux divergence).
-// BV: the base varies along the line (z); in x and y it is one value bc, and
-// the pair carries U itself: the base part's flux difference is then
+// BV: the base varies along the line (z): dif is the face's two rows of
+// base_rows, b its bases at c and c + 1.  In x and y it is one value bc, and the
+// pair carries U itself: the base part's flux difference is then
 // (U_c - U_{c-1}) * bc * rho, with the difference of two FP32 values exact
 // in FP64.
 struct SF32 {
@@ -162,7 +193,8 @@ struct PolicyF32 {
     static constexpr int kZWaves = 1;      // the z pass's registers as the compiler allocates them
     static constexpr bool kXVec = false;   // the x pass stays the row-staged kernel
     template <int O, bool BV>
-    static __device__ __forceinline__ SFlux scal_flux(const TC *win, const double *bwin, TC U, double rho) {
+    static __device__ __forceinline__ SFlux scal_flux(const TC *win, const float *dif, const double *b, TC U,
+                                                      double rho) {
         constexpr int R = Interp<O, float>::R;
         const bool pos = U >= 0.0f;
         // selects of values with constant indices (an index select would
@@ -171,13 +203,22 @@ struct PolicyF32 {
         float q[2 * R - 1];
         double bc = 0.0;
         if (BV) {
-            bc = pos ? bwin[R - 1] : bwin[R];
+            // the face's row of base differences and its base, of the upwind side
+            constexpr int ND = base_nd(R);
+            const int side = pos ? 0 : 1;
+            bc = b[side];
+            float d[ND];
 #pragma unroll
-            for (int m = 0; m < 2 * R - 1; ++m) {
-                const float wv = pos ? win[m] : win[2 * R - 1 - m];
-                const double bv = pos ? bwin[m] : bwin[2 * R - 1 - m];
-                q[m] = (wv - pc) + (float)(bv - bc);
+            for (int m = 0; m < ND; m += 4) {
+                const float4 v = *reinterpret_cast<const float4 *>(dif + side * ND + m);
+                d[m] = v.x;
+                d[m + 1] = v.y;
+                d[m + 2] = v.z;
+                d[m + 3] = v.w;
             }
+#pragma unroll
+            for (int m = 0; m < 2 * R - 1; ++m)
+                q[m] = m == R - 1 ? 0.0f : ((pos ? win[m] : win[2 * R - 1 - m]) - pc) + d[m < R - 1 ? m : m - 1];
         } else {
 #pragma unroll
             for (int m = 0; m < 2 * R - 1; ++m) q[m] = (pos ? win[m] : win[2 * R - 1 - m]) - pc;
@@ -277,8 +318,8 @@ __device__ __forceinline__ void rk_store(const Fields &fl, int v, unsigned o, un
 // tendencies and stage copies together after the fluxes; all unconditional,
 // so one counted wait covers each group.  The first face (k0 - 1, flux only)
 // is peeled off the loop.  The velocity and scalar windows are register
-// rings as in the y pass below; the scalars' FP64 base window, which is the
-// same for every lane and lives in scalar registers, shifts.
+// rings as in the y pass below.  FP32: a chunk holds at most ADV_Z_KMAX levels,
+// whose base rows are in LDS.
 template <class P, int SO, int MO, int NSC, bool MOM, int RKM>
 __global__ __launch_bounds__(256, P::kZWaves) void adv_z(Geo g, Prof pr, Fields fl, int kchunk) {
     using TS = typename P::TS;
@@ -295,10 +336,24 @@ __global__ __launch_bounds__(256, P::kZWaves) void adv_z(Geo g, Prof pr, Fields 
     const uint3 tile = xcd_tile<1>();  // XCD bands of 4-row blocks in y
     const int i = tile.x * 64 + threadIdx.x;
     const int j = tile.y * 4 + threadIdx.y;
-    if (i >= g.nx || j >= g.ny) return;  // no barriers in this kernel
     const int k0 = g.gw + tile.z * kchunk;
     const int k1 = min(k0 + kchunk, g.nz + g.gw);
     const int ktop = g.nzg - 1;
+    constexpr bool BASE = P::kBase && NSC > 0;
+    constexpr int NT = BASE ? ADV_Z_KMAX + 1 : 1;  // faces of a chunk
+    __shared__ __align__(16) float bdif[NS][NT][2][base_nd(RS)];
+    __shared__ double bpro[NS][NT + 1];  // bases at levels k0 - 1 .. k1
+    if (BASE) {
+        const int tid = threadIdx.y * 64 + threadIdx.x;
+        base_rows<RS, NS, NT>(fl, k0 - 1, k1 - k0 + 1, ktop, tid, 256, bdif);
+        for (int e = tid; e < NS * (k1 - k0 + 2); e += 256) {
+            const int sc = e / (k1 - k0 + 2), l = e % (k1 - k0 + 2);
+            const double *p = sc == 0 ? fl.base[0] : fl.base[1];
+            bpro[sc][l] = p ? p[min(k0 - 1 + l, ktop)] : 0.0;
+        }
+        __syncthreads();
+    }
+    if (i >= g.nx || j >= g.ny) return;  // no barriers from here on
     const unsigned plane = (unsigned)g.plane;
     const unsigned col = (unsigned)j * g.nx + i;
     const TS *ps[2] = {(const TS *)fl.q[0], (const TS *)fl.q[1]};
@@ -312,10 +367,8 @@ __global__ __launch_bounds__(256, P::kZWaves) void adv_z(Geo g, Prof pr, Fields 
         cx[m] = (unsigned)j * g.nx + wrapi(i + m - (RM - 2), g.nx);
         cy[m] = (unsigned)wrapi(j + m - (RM - 2), g.ny) * g.nx + i;
     }
-    auto base_at = [&](int sc, int lev) { return P::kBase ? (fl.base[sc] ? fl.base[sc][lev] : 0.0) : 0.0; };
     // windows of face c: level c - (R-1) + m in slot m (rings: phase 0)
     TC rs[NS][L];
-    double bw[NS][2 * RS];
     TC ru[L], rv[L], rw[L];
     TC cwx[NC], cwy[NC];  // w along x and y at level c
     int c = k0 - 1;
@@ -325,7 +378,6 @@ __global__ __launch_bounds__(256, P::kZWaves) void adv_z(Geo g, Prof pr, Fields 
         for (int m = 0; m < 2 * RS; ++m) {
             const int lev = c - (RS - 1) + m;
             rs[sc][m] = (TC)ld(ps[sc], lev * plane + col);
-            bw[sc][m] = base_at(sc, lev);
         }
     if (MOM) {
 #pragma unroll
@@ -348,14 +400,10 @@ __global__ __launch_bounds__(256, P::kZWaves) void adv_z(Geo g, Prof pr, Fields 
     };
     // next-face window loads, issued before the current face's arithmetic
     TC nws[NS], nu = 0, nv = 0, nw = 0;
-    double nbw[NS];
     auto issue_next = [&](int cc) {
         const int ls = min(cc + 1 + RS, ktop);
 #pragma unroll
-        for (int sc = 0; sc < NSC; ++sc) {
-            nws[sc] = (TC)ld(ps[sc], ls * plane + col);
-            nbw[sc] = base_at(sc, ls);
-        }
+        for (int sc = 0; sc < NSC; ++sc) nws[sc] = (TC)ld(ps[sc], ls * plane + col);
         if (MOM) {
             const unsigned o = (unsigned)min(cc + 1 + RM, ktop) * plane + col;
             nu = (TC)ld(pu, o);
@@ -364,15 +412,9 @@ __global__ __launch_bounds__(256, P::kZWaves) void adv_z(Geo g, Prof pr, Fields 
         }
     };
     // the next levels into the rings' free slots (phase PH), or, without
-    // rings, the windows shifted; the base window always shifts
+    // rings, the windows shifted
     auto advance = [&](auto phc) {
         constexpr int PH = RING ? decltype(phc)::value : 0;
-#pragma unroll
-        for (int sc = 0; sc < NSC; ++sc) {
-#pragma unroll
-            for (int m = 0; m < WS - 1; ++m) bw[sc][m] = bw[sc][m + 1];
-            bw[sc][WS - 1] = nbw[sc];
-        }
         if (RING) {
 #pragma unroll
             for (int sc = 0; sc < NSC; ++sc) rs[sc][(WS + PH) % L] = nws[sc];
@@ -424,7 +466,10 @@ __global__ __launch_bounds__(256, P::kZWaves) void adv_z(Geo g, Prof pr, Fields 
         const double rho0c = pr.rho0[cc];
         const TC W = MOM ? wsw[RM - 1] : (TC)ld(pw, (unsigned)cc * plane + col);
 #pragma unroll
-        for (int sc = 0; sc < NSC; ++sc) F[sc] = P::template scal_flux<SO, true>(ws[sc], bw[sc], W, rho0c);
+        for (int sc = 0; sc < NSC; ++sc) {
+            const int f = BASE ? cc - (k0 - 1) : 0;
+            F[sc] = P::template scal_flux<SO, true>(ws[sc], bdif[sc][f][0], bpro[sc] + f, W, rho0c);
+        }
         if (MOM) {
             // u advected by w: U = centred(w along x), rho0[k]
             Fu_ = P::template mom_flux<MO>(wsu, Interp<MO, TC>::centred(cwx), rho0c);
@@ -648,7 +693,7 @@ __global__ __launch_bounds__(256) void adv_y(Geo g, Prof pr, Fields fl, int jchu
         TC &Fw_ = FIRST ? Fw_prev : Fw;
         const TC V = MOM ? wsv[RM - 1] : (TC)ld(pv, orow);
 #pragma unroll
-        for (int sc = 0; sc < NSC; ++sc) F[sc] = P::template scal_flux<SO, false>(ws[sc], bw[sc], V, rh);
+        for (int sc = 0; sc < NSC; ++sc) F[sc] = P::template scal_flux<SO, false>(ws[sc], nullptr, bw[sc], V, rh);
         // the scalar fluxes cover the latency of the centred stencil loads
         __builtin_amdgcn_sched_barrier(0);
         if (MOM) {
@@ -761,6 +806,7 @@ __global__ __launch_bounds__(64 * TY, P::kYZWaves) void adv_yz(Geo g, Prof pr, F
     constexpr int NXH = (2 * TY + 1) * (NC - 1);         // x halo items (v: TY + 1 rows, w: TY rows)
     constexpr int NPL = ADV_YZ_KMAX + 2 * R;             // profile levels k0 - R .. k0 + kchunk + R - 1
     constexpr int NPR = P::kBase ? 4 + NSC : 4;
+    constexpr int NT = P::kBase ? ADV_YZ_KMAX + 1 : 1;   // faces k0 - 1 .. of base_rows
     static_assert(NXH <= 64 * TY, "x halo items exceed the block");
     // tile and face fluxes double-buffered by level parity: level c + 1 is
     // staged while slower waves still read level c, so one barrier per face
@@ -768,6 +814,7 @@ __global__ __launch_bounds__(64 * TY, P::kYZWaves) void adv_yz(Geo g, Prof pr, F
     __shared__ TC flx[2][NV][TY + 1][64];  // y flux of face j0 - 1 + f + 1/2 in slot f
     __shared__ TC vring[NR][64];           // v of row j0 - 1 at level lev in slot lev % NR
     __shared__ double lp[NPR][NPL];        // rho0, rho0_half, alpha0, alpha0_half (, scalar bases)
+    __shared__ __align__(16) float bdif[NSC][NT][2][base_nd(R)];
     const uint3 tl = xcd_tile<1>();        // XCD bands of TY-row blocks in y
     const int tx = threadIdx.x, ty = threadIdx.y;
     const int nx = g.nx, ny = g.ny;
@@ -795,6 +842,7 @@ __global__ __launch_bounds__(64 * TY, P::kYZWaves) void adv_yz(Geo g, Prof pr, F
             for (int sc = 0; sc < NSC; ++sc) lp[(4 + sc) % NPR][l] = fl.base[sc] ? fl.base[sc][lev] : 0.0;
         }
     }
+    if (P::kBase) base_rows<R, NSC, NT>(fl, k0 - 1, k1 - k0 + 1, ktop, ty * 64 + tx, 64 * TY, bdif);
     auto prof = [&](int q, int lev) { return lp[q][lev - kb]; };
     const TS *pf[NV];
 #pragma unroll
@@ -902,12 +950,9 @@ __global__ __launch_bounds__(64 * TY, P::kYZWaves) void adv_yz(Geo g, Prof pr, F
             }
             const double rho0c = prof(0, c);
 #pragma unroll
-            for (int sc = 0; sc < NSC; ++sc) {
-                double bz[WN];
-#pragma unroll
-                for (int m = 0; m < WN; ++m) bz[m] = P::kBase ? prof((4 + sc) % NPR, c - (R - 1) + m) : 0.0;
-                Fs[sc] = P::template scal_flux<SO, true>(rs[sc], bz, rw[R - 1], rho0c);
-            }
+            for (int sc = 0; sc < NSC; ++sc)
+                Fs[sc] = P::template scal_flux<SO, true>(rs[sc], bdif[sc][P::kBase ? c - (k0 - 1) : 0][0],
+                                                         &lp[(4 + sc) % NPR][c - kb], rw[R - 1], rho0c);
             Fu = P::template mom_flux<MO>(ru, Interp<MO, TC>::centred(cwx), rho0c);
             Fv = P::template mom_flux<MO>(rv, Interp<MO, TC>::centred(cwy), rho0c);
             TC q[NC];
@@ -928,8 +973,7 @@ __global__ __launch_bounds__(64 * TY, P::kYZWaves) void adv_yz(Geo g, Prof pr, F
                 for (int m = 0; m < WN; ++m) win[m] = tile[b][v][ty + 1 + m][XL + tx];
                 TC q[NC];
                 if (v < NSC) {
-                    const double bdum[WN] = {};
-                    Fy[v] = P::x_keep(P::template scal_flux<SO, false>(win, bdum, Vc, rh));
+                    Fy[v] = P::x_keep(P::template scal_flux<SO, false>(win, nullptr, nullptr, Vc, rh));
                 } else if (v == FU) {
 #pragma unroll
                     for (int m = 0; m < NC; ++m) q[m] = tile[b][FV][R + ty][tx + m];  // v along x
@@ -953,8 +997,7 @@ __global__ __launch_bounds__(64 * TY, P::kYZWaves) void adv_yz(Geo g, Prof pr, F
                 for (int m = 0; m < WN; ++m) win[m] = tile[b][ev][m][XL + tx];
                 TC F;
                 if (ev < NSC) {
-                    const double bdum[WN] = {};
-                    F = P::x_keep(P::template scal_flux<SO, false>(win, bdum, tile[b][FV][R - 1][XL + tx], rh));
+                    F = P::x_keep(P::template scal_flux<SO, false>(win, nullptr, nullptr, tile[b][FV][R - 1][XL + tx], rh));
                 } else if (ev == FU) {
 #pragma unroll
                     for (int m = 0; m < NC; ++m) q[m] = tile[b][FV][R - 1][tx + m];
@@ -1214,7 +1257,7 @@ __global__ __launch_bounds__(256) void adv_x(Geo g, Prof pr, Fields fl) {
             TC win[2 * RS];
 #pragma unroll
             for (int m = 0; m < 2 * RS; ++m) win[m] = srow[c - (RS - 1) + m];
-            flux[sc * nx + c] = P::x_keep(P::template scal_flux<SO, false>(win, bw[sc], urow[c], rh));
+            flux[sc * nx + c] = P::x_keep(P::template scal_flux<SO, false>(win, nullptr, bw[sc], urow[c], rh));
         }
         if (MOM) {
 #pragma unroll
@@ -1397,7 +1440,8 @@ __global__ __launch_bounds__(P::kXThreads, SO == 5 && MO == 5 ? P::kXWaves5 : 1)
 #pragma unroll
         for (int e = 0; e < C; ++e)
             if (e >= lo && e < hi)
-                F[sc][e] = P::x_keep(P::template scal_flux<SO, false>(xs[sc] + X0 + e - (RS - 1), bw[sc], xu[X0 + e], rh));
+                F[sc][e] = P::x_keep(P::template scal_flux<SO, false>(xs[sc] + X0 + e - (RS - 1), nullptr, bw[sc], xu[X0 + e],
+                                                                   rh));
     };
     auto momentum = [&](int lo, int hi) {  // advected component u, v, w
 #pragma unroll

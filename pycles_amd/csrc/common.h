@@ -107,17 +107,21 @@ static inline ZSplit adv_zsplit(int n, long long cols) {
     }
     return best;
 }
-// The advection y pass's chunks of the ny rows and the z pass's chunks of the
-// interior levels.
+// The advection y pass's chunks of the ny rows.
 static inline ZSplit advy_zsplit(int nx, int ny, int nz) {
     return adv_zsplit(ny, (long long)((nx + 63) / 64) * ((nz + 3) / 4));
 }
+// The z pass's chunks of the interior levels, none longer than ADV_Z_KMAX (the LDS rows of the FP32 form's
+// profile differences).
+constexpr int ADV_Z_KMAX = 128;
 static inline ZSplit advz_zsplit(int nx, int ny, int nz) {
-    return adv_zsplit(nz, (long long)((nx + 63) / 64) * ((ny + 3) / 4));
+    const ZSplit z = adv_zsplit(nz, (long long)((nx + 63) / 64) * ((ny + 3) / 4));
+    return z.len > ADV_Z_KMAX ? zsplit_ceil(nz, (nz + ADV_Z_KMAX - 1) / ADV_Z_KMAX) : z;
 }
 // The fused y-z advection pass: the z pass's chunks, none longer than
-// ADV_YZ_KMAX levels (the LDS copy of a chunk's level profiles holds that many).
-constexpr int ADV_YZ_KMAX = 128;
+// ADV_YZ_KMAX levels (the LDS copies of a chunk's level profiles and their
+// differences hold that many; three FP32 blocks of 52 KB fit a CU).
+constexpr int ADV_YZ_KMAX = 96;
 static inline ZSplit advyz_zsplit(int nx, int ny, int nz) {
     const ZSplit z = advz_zsplit(nx, ny, nz);
     return z.len > ADV_YZ_KMAX ? zsplit_ceil(nz, (nz + ADV_YZ_KMAX - 1) / ADV_YZ_KMAX) : z;

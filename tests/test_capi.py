@@ -142,3 +142,13 @@ def test_layout_and_cfl_read_reject_bad_arguments(lib):
     assert lib.pycles_layout_egress(C.byref(d), fake, fake, None, -1, None) == -1
     assert lib.pycles_cfl_read(None, None, None) == -1
     assert lib.pycles_launch_chunks(9, C.byref(d), C.byref(C.c_int()), C.byref(C.c_int())) == -1
+
+
+def test_advection_z_chunks_fit_their_lds_rows(lib):
+    """No z chunk of the advection is longer than what the FP32 kernels keep
+    in LDS for it: 128 levels in the z pass, 96 in the fused y-z pass."""
+    for plane in ((64, 64), (8, 8), (1024, 512), (2048, 1024), (30000, 8)):
+        for nz in (3, 75, 96, 97, 128, 129, 192, 255, 511, 1000):
+            for kern, cap in ((2, 128), (4, 96)):
+                nch, ln = _chunks(lib, kern, plane + (nz,))
+                assert ln <= cap and nch * ln >= nz and (nch - 1) * ln < nz, (kern, plane, nz, nch, ln)
