@@ -249,54 +249,25 @@ template <typename T> __device__ __forceinline__ T sq_eps(T b) {
 
 template <int ORDER, typename T> struct Interp;
 
-// A WENO smoothness indicator as a sum of squares, for the FP32 form at orders
-// 7 and 9.  c holds the reference's coefficients of q[i] q[j], i <= j, row by
-// row, without the centre's, which is zero there; with the symmetric matrix
-// they stand for factored as L D L^T, the indicator is
-//   sum over i of d[i] (q[i] + sum over j > i of l[i][j] q[j])^2.
-// As many operations as the nested form (14 at order 9), but its terms do not
-// cancel: the nested form loses three digits of the indicator in FP32, and
-// with them a reconstruction of noise errs by 2.6e-7 of it (rms, order 9;
-// 0.9e-7 at order 7) against 0.5e-7 (0.4e-7).
-template <int N> struct Squares {
-    double d[N] = {}, l[N][N] = {};
-    constexpr Squares(const double (&c)[N * (N + 1) / 2]) {
-        double a[N][N] = {};
-        int t = 0;
-        for (int i = 0; i < N; ++i)
-            for (int j = i; j < N; ++j) a[i][j] = j == i ? c[t++] : 0.5 * c[t++];
-        for (int i = 0; i < N; ++i) {
-            d[i] = a[i][i];
-            for (int j = i + 1; j < N; ++j) l[i][j] = a[i][j] / d[i];
-            for (int m = i + 1; m < N; ++m)
-                for (int j = m; j < N; ++j) a[m][j] -= d[i] * l[i][m] * l[i][j];
-        }
-    }
-};
-template <int N, typename T> __device__ __forceinline__ T sum_squares(const Squares<N> &s, const T (&q)[N]) {
-    T b = T(0);
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-        T y = q[i];
-#pragma unroll
-        for (int j = i + 1; j < N; ++j) y += T(s.l[i][j]) * q[j];
-        b = i == 0 ? (T(s.d[i]) * y) * y : b + (T(s.d[i]) * y) * y;
-    }
-    return b;
+// Correctly rounded multiply and add that are never contracted into an FMA
+// (the pragma drops the contraction permission from these operations), so an
+// expression gives the same bits in every translation unit whatever its
+// contraction flag.
+__device__ __forceinline__ double mul_rn(double a, double b) {
+#pragma clang fp contract(off)
+    return a * b;
 }
-// The weighted mean of N candidates from s[k], candidate k times its linear
-// weight d[k], and the smoothness indicators b[k]: two multiply-add chains
-// over r_k = 1 / (b_k + eps)^2 and one final reciprocal.
-template <int N, typename T> __device__ __forceinline__ T weno_mean(const T (&s)[N], const T (&b)[N], const double (&d)[N]) {
-    T num = T(0), den = T(0);
-#pragma unroll
-    for (int k = 0; k < N; ++k) {
-        const T t = b[k] + T(1e-10);
-        const T r = Num<T>::rcp(t * t);
-        num = k == 0 ? s[k] * r : num + s[k] * r;
-        den = k == 0 ? T(d[k]) * r : den + T(d[k]) * r;
-    }
-    return num * Num<T>::rcp(den);
+__device__ __forceinline__ double add_rn(double a, double b) {
+#pragma clang fp contract(off)
+    return a + b;
+}
+__device__ __forceinline__ float mul_rn(float a, float b) {
+#pragma clang fp contract(off)
+    return a * b;
+}
+__device__ __forceinline__ float add_rn(float a, float b) {
+#pragma clang fp contract(off)
+    return a + b;
 }
 
 template <typename T> struct Interp<5, T> {
@@ -327,6 +298,13 @@ template <typename T> struct Interp<5, T> {
     // common factor), and the weighted sum and the sum of the weights are two
     // multiply-add chains over r_k = 1 / (4 b_k + 4 eps)^2 with one final
     // reciprocal: 34 operations and 4 reciprocals against 43 and 4.
+    // Indicators as sums of squares, (16/3) (m2 - (19/8) m1)^2 + (13/4) m1^2 and
+    // so on, take 23 and 4 and are a little more exact, and the step at 512 x 512
+    // x 256 3% less time; but the velocities' last bits return in
+    // the entropy's tendency, s div(rho u), thousands of times the net one, so
+    // that other roundings of the fluxes, more exact or not, move the entropy
+    // after one step by up to 3e-5 of its deviations, which FP32 velocities
+    // leave undetermined.  The form's bits are kept instead.
     static __device__ __forceinline__ T weno_c0(const T *q) {
         const T m2 = q[0], m1 = q[1], p1 = q[3], p2 = q[4];
         const T s0 = T(0.1 / 3.0) * m2 - T(0.7 / 6.0) * m1;  // 0.1 ((1/3) m2 - (7/6) m1)
@@ -378,20 +356,33 @@ template <typename T> struct Interp<7, T> {
         const T w0 = a0 * inv, w1 = a1 * inv, w2 = a2 * inv, w3 = a3 * inv;
         return w0 * s0 + w1 * s1 + w2 * s2 + w3 * s3;
     }
-    // weno() of a stencil whose centre value q[3] is zero, for the FP32 form
-    // (see order 9): 68 operations and 5 reciprocals against 108 and 5.
+    // weno() of a stencil whose centre value q[3] is zero (offsets from the
+    // centre), for the FP32 form: without the centre's terms, 79 operations and
+    // 5 reciprocals against 108 and 5, and the same bits: where a centre's term
+    // was the partner of a product in a multiply-add, mul_rn leaves that product
+    // rounded by itself.  200 x 135 x 75 WENO7 tendencies 185 -> 159 us, with the
+    // profile rows of the z pass (advection_impl.h).
     static __device__ __forceinline__ T weno_c0(const T *q) {
-        constexpr double d[4] = {1.0 / 35.0, 12.0 / 35.0, 18.0 / 35.0, 4.0 / 35.0};
-        constexpr Squares<3> outer({547.0, -3882.0, 4642.0, 7043.0, -17246.0, 11003.0});
-        constexpr Squares<3> inner({267.0, -1642.0, -494.0, 2843.0, 1922.0, 547.0});
         const T m3 = q[0], m2 = q[1], m1 = q[2], p1 = q[4], p2 = q[5], p3 = q[6];
-        const T s[4] = {T(-0.25 * d[0]) * m3 + T(13.0 / 12.0 * d[0]) * m2 - T(23.0 / 12.0 * d[0]) * m1,
-                        T(1.0 / 12.0 * d[1]) * m2 - T(5.0 / 12.0 * d[1]) * m1 + T(0.25 * d[1]) * p1,
-                        T(-1.0 / 12.0 * d[2]) * m1 + T(7.0 / 12.0 * d[2]) * p1 - T(1.0 / 12.0 * d[2]) * p2,
-                        T(13.0 / 12.0 * d[3]) * p1 - T(5.0 / 12.0 * d[3]) * p2 + T(1.0 / 12.0 * d[3]) * p3};
-        const T b[4] = {sum_squares<3, T>(outer, {m3, m2, m1}), sum_squares<3, T>(inner, {m2, m1, p1}),
-                        sum_squares<3, T>(inner, {p2, p1, m1}), sum_squares<3, T>(outer, {p3, p2, p1})};
-        return weno_mean<4, T>(s, b, d);
+        const T s0 = T(-1.0 / 4.0) * m3 + T(13.0 / 12.0) * m2 + T(-23.0 / 12.0) * m1;
+        const T s1 = T(1.0 / 12.0) * m2 + T(-5.0 / 12.0) * m1 + T(1.0 / 4.0) * p1;
+        const T s2 = mul_rn(T(-1.0 / 12.0), m1) + T(7.0 / 12.0) * p1 + T(-1.0 / 12.0) * p2;
+        const T s3 = mul_rn(T(13.0 / 12.0), p1) + T(-5.0 / 12.0) * p2 + T(1.0 / 12.0) * p3;
+        const T b0 = m3 * (T(547.0) * m3 - T(3882.0) * m2 + T(4642.0) * m1) + m2 * (T(7043.0) * m2 - T(17246.0) * m1) +
+                     m1 * mul_rn(T(11003.0), m1);
+        const T b1 = m2 * (T(267.0) * m2 - T(1642.0) * m1 - T(494.0) * p1) + m1 * (mul_rn(T(2843.0), m1) + T(1922.0) * p1) +
+                     T(547.0) * p1 * p1;
+        const T b2 = mul_rn(m1, mul_rn(T(547.0), m1) + T(1922.0) * p1 - T(494.0) * p2) +
+                     p1 * (T(2843.0) * p1 - T(1642.0) * p2) + T(267.0) * p2 * p2;
+        const T b3 = mul_rn(p1, T(11003.0) * p1 - T(17246.0) * p2 + T(4642.0) * p3) + p2 * (T(7043.0) * p2 - T(3882.0) * p3) +
+                     T(547.0) * p3 * p3;
+        const T a0 = Num<T>::div(T(1.0 / 35.0), sq_eps(b0));
+        const T a1 = Num<T>::div(T(12.0 / 35.0), sq_eps(b1));
+        const T a2 = Num<T>::div(T(18.0 / 35.0), sq_eps(b2));
+        const T a3 = Num<T>::div(T(4.0 / 35.0), sq_eps(b3));
+        const T inv = Num<T>::rcp(a0 + a1 + a2 + a3);
+        const T w0 = a0 * inv, w1 = a1 * inv, w2 = a2 * inv, w3 = a3 * inv;
+        return w0 * s0 + w1 * s1 + w2 * s2 + w3 * s3;
     }
     // interp_6: q = phim2 .. phip3
     static __device__ __forceinline__ T centred(const T *q) {
@@ -439,28 +430,40 @@ template <typename T> struct Interp<9, T> {
         const T w0 = a0 * inv, w1 = a1 * inv, w2 = a2 * inv, w3 = a3 * inv, w4 = a4 * inv;
         return w0 * s0 + w1 * s1 + w2 * s2 + w3 * s3 + w4 * s4;
     }
-    // weno() of a stencil whose centre value q[4] is zero (offsets from the
-    // centre), for the FP32 form, rearranged like order 5's: the centre's terms
-    // dropped, the linear weights folded into the candidates, the indicators
-    // as sums of squares: 116 operations and 6 reciprocals against 174 and 6.
+    // weno() of a stencil whose centre value q[4] is zero, without its terms
+    // (see order 7): 129 operations and 6 reciprocals against 174 and 6, the same
+    // bits.  1024 x 1024 x 192 WENO9/5 tendencies 12.3 -> 11.3 ms, with the profile
+    // rows.
     static __device__ __forceinline__ T weno_c0(const T *q) {
-        constexpr double d[5] = {1.0 / 126.0, 10.0 / 63.0, 10.0 / 21.0, 20.0 / 63.0, 5.0 / 126.0};
-        constexpr Squares<4> outer({22658.0, -208501.0, 364863.0, -288007.0, 482963.0, -1704396.0, 1358458.0, 1521393.0,
-                                    -2462076.0, 1020563.0});
-        constexpr Squares<4> inner({6908.0, -60871.0, 99213.0, 18079.0, 138563.0, -464976.0, -88297.0, 406293.0,
-                                    165153.0, 22658.0});
-        constexpr Squares<4> middle({6908.0, -51001.0, -38947.0, 8209.0, 104963.0, 179098.0, -38947.0, 104963.0,
-                                     -51001.0, 6908.0});
         const T m4 = q[0], m3 = q[1], m2 = q[2], m1 = q[3], p1 = q[5], p2 = q[6], p3 = q[7], p4 = q[8];
-        const T s[5] = {T(0.2 * d[0]) * m4 - T(1.05 * d[0]) * m3 + T(137.0 / 60.0 * d[0]) * m2 - T(163.0 / 60.0 * d[0]) * m1,
-                        T(-0.05 * d[1]) * m3 + T(17.0 / 60.0 * d[1]) * m2 - T(43.0 / 60.0 * d[1]) * m1 + T(0.2 * d[1]) * p1,
-                        T(1.0 / 30.0 * d[2]) * m2 - T(13.0 / 60.0 * d[2]) * m1 + T(0.45 * d[2]) * p1 - T(0.05 * d[2]) * p2,
-                        T(-0.05 * d[3]) * m1 + T(47.0 / 60.0 * d[3]) * p1 - T(13.0 / 60.0 * d[3]) * p2 + T(1.0 / 30.0 * d[3]) * p3,
-                        T(77.0 / 60.0 * d[4]) * p1 - T(43.0 / 60.0 * d[4]) * p2 + T(17.0 / 60.0 * d[4]) * p3 - T(0.05 * d[4]) * p4};
-        const T b[5] = {sum_squares<4, T>(outer, {m4, m3, m2, m1}), sum_squares<4, T>(inner, {m3, m2, m1, p1}),
-                        sum_squares<4, T>(middle, {m2, m1, p1, p2}), sum_squares<4, T>(inner, {p3, p2, p1, m1}),
-                        sum_squares<4, T>(outer, {p4, p3, p2, p1})};
-        return weno_mean<5, T>(s, b, d);
+        const T s0 = T(1.0 / 5.0) * m4 + T(-21.0 / 20.0) * m3 + T(137.0 / 60.0) * m2 + T(-163.0 / 60.0) * m1;
+        const T s1 = T(-1.0 / 20.0) * m3 + T(17.0 / 60.0) * m2 + T(-43.0 / 60.0) * m1 + T(1.0 / 5.0) * p1;
+        const T s2 = T(1.0 / 30.0) * m2 + T(-13.0 / 60.0) * m1 + T(9.0 / 20.0) * p1 + T(-1.0 / 20.0) * p2;
+        const T s3 = mul_rn(T(-1.0 / 20.0), m1) + T(47.0 / 60.0) * p1 + T(-13.0 / 60.0) * p2 + T(1.0 / 30.0) * p3;
+        const T s4 = mul_rn(T(77.0 / 60.0), p1) + T(-43.0 / 60.0) * p2 + T(17.0 / 60.0) * p3 + T(-1.0 / 20.0) * p4;
+        const T b0 = m4 * (T(22658.0) * m4 - T(208501.0) * m3 + T(364863.0) * m2 - T(288007.0) * m1) +
+                     m3 * (T(482963.0) * m3 - T(1704396.0) * m2 + T(1358458.0) * m1) +
+                     m2 * (T(1521393.0) * m2 - T(2462076.0) * m1) + m1 * mul_rn(T(1020563.0), m1);
+        const T b1 = m3 * (T(6908.0) * m3 - T(60871.0) * m2 + T(99213.0) * m1 + T(18079.0) * p1) +
+                     m2 * (T(138563.0) * m2 - T(464976.0) * m1 - T(88297.0) * p1) +
+                     m1 * (mul_rn(T(406293.0), m1) + T(165153.0) * p1) + T(22658.0) * p1 * p1;
+        const T b2 = m2 * (T(6908.0) * m2 - T(51001.0) * m1 - T(38947.0) * p1 + T(8209.0) * p2) +
+                     m1 * (mul_rn(T(104963.0), m1) + T(179098.0) * p1 - T(38947.0) * p2) +
+                     p1 * (T(104963.0) * p1 - T(51001.0) * p2) + T(6908.0) * p2 * p2;
+        const T b3 = mul_rn(m1, mul_rn(T(22658.0), m1) + T(165153.0) * p1 - T(88297.0) * p2 + T(18079.0) * p3) +
+                     p1 * (T(406293.0) * p1 - T(464976.0) * p2 + T(99213.0) * p3) +
+                     p2 * (T(138563.0) * p2 - T(60871.0) * p3) + T(6908.0) * p3 * p3;
+        const T b4 = mul_rn(p1, T(1020563.0) * p1 - T(2462076.0) * p2 + T(1358458.0) * p3 - T(288007.0) * p4) +
+                     p2 * (T(1521393.0) * p2 - T(1704396.0) * p3 + T(364863.0) * p4) +
+                     p3 * (T(482963.0) * p3 - T(208501.0) * p4) + T(22658.0) * p4 * p4;
+        const T a0 = Num<T>::div(T(1.0 / 126.0), sq_eps(b0));
+        const T a1 = Num<T>::div(T(10.0 / 63.0), sq_eps(b1));
+        const T a2 = Num<T>::div(T(10.0 / 21.0), sq_eps(b2));
+        const T a3 = Num<T>::div(T(20.0 / 63.0), sq_eps(b3));
+        const T a4 = Num<T>::div(T(5.0 / 126.0), sq_eps(b4));
+        const T inv = Num<T>::rcp(a0 + a1 + a2 + a3 + a4);
+        const T w0 = a0 * inv, w1 = a1 * inv, w2 = a2 * inv, w3 = a3 * inv, w4 = a4 * inv;
+        return w0 * s0 + w1 * s1 + w2 * s2 + w3 * s3 + w4 * s4;
     }
     // interp_8: q = phim3 .. phip4
     static __device__ __forceinline__ T centred(const T *q) {
@@ -468,36 +471,6 @@ template <typename T> struct Interp<9, T> {
                 T(29.0 / 840.0) * (q[1] + q[6]) - T(1.0 / 280.0) * (q[0] + q[7]));
     }
 };
-
-// Upwinded face flux through the face between stencil cells R-1 and R of
-// win[0 .. 2R-1] (win[m] = phi at face-cell offset m-(R-1)).
-//
-// The reference evaluates both one-sided reconstructions and blends them as
-// 0.5*((U+|U|)*phi_p + (U-|U|)*phi_m)*rho (scalar_advection.h:361).  For
-// finite U and phi that equals U*phi_p*rho when U >= 0 and U*phi_m*rho when
-// U < 0 to the last bit: (U+|U|) = 2U and (U-|U|) = 0 exactly, 2U*phi rounds
-// to twice fl(U*phi), and the 0.5 scaling is exact.  So the kernels select the
-// upwind stencil first and evaluate one reconstruction per face.
-// Correctly rounded multiply and add that are never contracted into an FMA
-// (the pragma drops the contraction permission from these operations), so an
-// expression gives the same bits in every translation unit whatever its
-// contraction flag.
-__device__ __forceinline__ double mul_rn(double a, double b) {
-#pragma clang fp contract(off)
-    return a * b;
-}
-__device__ __forceinline__ double add_rn(double a, double b) {
-#pragma clang fp contract(off)
-    return a + b;
-}
-__device__ __forceinline__ float mul_rn(float a, float b) {
-#pragma clang fp contract(off)
-    return a * b;
-}
-__device__ __forceinline__ float add_rn(float a, float b) {
-#pragma clang fp contract(off)
-    return a + b;
-}
 
 // TimeStepping.update_third (TimeStepping.pyx:131-151), one point of stage RK:
 // phi is the value, tn its tendency, cp the stage-0 copy.  Uncontracted, in
@@ -510,6 +483,15 @@ __device__ __forceinline__ T rk_update(T phi, T tn, T cp, T dt) {
     return add_rn(mul_rn(T(1.0 / 3.0), cp), mul_rn(T(2.0 / 3.0), x));
 }
 
+// Upwinded face flux through the face between stencil cells R-1 and R of
+// win[0 .. 2R-1] (win[m] = phi at face-cell offset m-(R-1)).
+//
+// The reference evaluates both one-sided reconstructions and blends them as
+// 0.5*((U+|U|)*phi_p + (U-|U|)*phi_m)*rho (scalar_advection.h:361).  For
+// finite U and phi that equals U*phi_p*rho when U >= 0 and U*phi_m*rho when
+// U < 0 to the last bit: (U+|U|) = 2U and (U-|U|) = 0 exactly, 2U*phi rounds
+// to twice fl(U*phi), and the 0.5 scaling is exact.  So the kernels select the
+// upwind stencil first and evaluate one reconstruction per face.
 template <int ORDER, typename T>
 __device__ __forceinline__ T upwind_flux(const T *win, T U, T rho) {
     constexpr int R = Interp<ORDER, T>::R;
