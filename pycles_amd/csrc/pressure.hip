@@ -193,7 +193,14 @@ __device__ __forceinline__ void stockham_fft(C2<T> *buf, int S, int b, int t, in
 // separated into the two half spectra.
 // TR: the spectrum as planes [kx][level][y] (plane_solve_kernel) instead of rows
 // [level][y][kx]; the block's 2S rows are then consecutive.
-template <typename TS, bool TR>
+// V consecutive cells per access (16 bytes; 1 where a field is off a 16-byte
+// boundary): a third of the addresses and more bytes in flight per thread than
+// with single cells, 512 x 512 x 256 FP64 560 -> 467 us (4.6 TB/s), FP32 267 ->
+// 250.  The phases of the few blocks that fit a CU bound it (memory, then LDS:
+// the real values' writes meet in a few banks).  Neighbouring lanes on 8
+// neighbouring rows have no such conflicts, but a row's share is then 128 bytes
+// and the memory slower (562 and 329).
+template <typename TS, bool TR, int V>
 __global__ __launch_bounds__(512) void div_fftx_kernel(Geo g, const TS *u, const TS *v, const TS *w,
                                                        const double *alpha0, const double *alpha0_half,
                                                        const double *partial, double *mean, double *cfl, TS *div_out,
@@ -233,58 +240,65 @@ __global__ __launch_bounds__(512) void div_fftx_kernel(Geo g, const TS *u, const
         if (kk == 0 && cfl) *cfl = 0.0;
     }
     const double dxi0 = 1.0 / g.dx[0], dxi1 = 1.0 / g.dx[1], dxi2 = 1.0 / g.dx[2];
-    // four cells per thread at a time: all their loads are issued before the
-    // arithmetic and the stores (a store in between would hold back the
-    // next cell's loads, which the compiler must assume it aliases)
-    const int B = blockDim.x, nt = g.nx << (logS + 1);
-    for (int t0 = threadIdx.x; t0 < nt; t0 += 4 * B) {
-        TS uc[4], um[4], vc[4], vm[4], wc[4], wm[4];
-        long long oo[4];
+    // Q accesses per field and thread at a time: all their loads are issued
+    // before the arithmetic and the stores (a store in between would hold back
+    // the next cells' loads, which the compiler must assume it aliases)
+    typedef TS VT __attribute__((ext_vector_type(V)));
+    constexpr int Q = V == 1 ? 4 : 2, LV = V == 1 ? 0 : (V == 2 ? 1 : 2);
+    const int B = blockDim.x, nt = (g.nx / V) << (logS + 1);
+    auto get = [](const TS *f) { return *reinterpret_cast<const VT *>(f); };
+    for (int t0 = threadIdx.x; t0 < nt; t0 += Q * B) {
+        VT uc[Q], vc[Q], vm[Q], wc[Q], wm[Q];
+        TS ue[Q];  // u of the cell before the first
+        long long oo[Q];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
+        for (int q = 0; q < Q; ++q) {
             const int t = min(t0 + q * B, nt - 1);  // a clamped duplicate past the end: loaded, not stored
-            const int i = t & (g.nx - 1);
-            const int j = j0 + (t >> logx);
+            const int i = (t & (g.nx / V - 1)) * V;
+            const int j = j0 + (t >> (logx - LV));
             const int jm = j == 0 ? g.ny - 1 : j - 1;
-            const int im1 = i == 0 ? g.nx - 1 : i - 1;
-            const long long o = gidx(g, i, j, k);
+            const long long row = gidx(g, 0, j, k), o = row + i;
             oo[q] = o;
-            uc[q] = u[o];
-            um[q] = u[gidx(g, im1, j, k)];
-            vc[q] = v[o];
-            vm[q] = v[gidx(g, i, jm, k)];
-            wc[q] = w[o];
-            wm[q] = w[o - g.plane];
+            uc[q] = get(u + o);
+            ue[q] = u[row + (i == 0 ? g.nx - 1 : i - 1)];
+            vc[q] = get(v + o);
+            vm[q] = get(v + gidx(g, i, jm, k));
+            wc[q] = get(w + o);
+            wm[q] = get(w + o - g.plane);
         }
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
+        for (int q = 0; q < Q; ++q) {
             const int t = t0 + q * B;
             if (t >= nt) continue;
-            const int i = t & (g.nx - 1);
-            const int rb = t >> logx;
-            TS d;
-            if (sizeof(TS) == 8) {
-                // the profiles are positive normal numbers: div64 is the
-                // IEEE quotient (common.h)
-                double dv = 0.0;
-                dv += (div64((double)uc[q], ah) - div64((double)um[q], ah)) * dxi0;
-                dv += (div64((double)vc[q], ah) - div64((double)vm[q], ah)) * dxi1;
-                const double wk = (double)wc[q] - mk;
-                const double wkm = (double)wm[q] - mkm;
-                dv += (div64(wk, a0) - div64(wkm, a0m)) * dxi2;
-                d = (TS)dv;
-            } else {
-                // FP32 path: rho0*u in FP32 except the level means and profiles
-                const float rh = (float)(1.0 / ah);
-                float dv = ((float)uc[q] - (float)um[q]) * (float)(dxi0)*rh;
-                dv += ((float)vc[q] - (float)vm[q]) * (float)(dxi1)*rh;
-                const float wk = (float)((double)wc[q] - mk);
-                const float wkm = (float)((double)wm[q] - mkm);
-                dv += (wk * (float)(1.0 / a0) - wkm * (float)(1.0 / a0m)) * (float)dxi2;
-                d = (TS)dv;
+            const int i = (t & (g.nx / V - 1)) * V, rb = t >> (logx - LV);
+            VT d;
+            TS um = ue[q];
+#pragma unroll
+            for (int e = 0; e < V; ++e) {
+                if (sizeof(TS) == 8) {
+                    // the profiles are positive normal numbers: div64 is the
+                    // IEEE quotient (common.h)
+                    double dv = 0.0;
+                    dv += (div64((double)uc[q][e], ah) - div64((double)um, ah)) * dxi0;
+                    dv += (div64((double)vc[q][e], ah) - div64((double)vm[q][e], ah)) * dxi1;
+                    const double wk = (double)wc[q][e] - mk;
+                    const double wkm = (double)wm[q][e] - mkm;
+                    dv += (div64(wk, a0) - div64(wkm, a0m)) * dxi2;
+                    d[e] = (TS)dv;
+                } else {
+                    // FP32 path: rho0*u in FP32 except the level means and profiles
+                    const float rh = (float)(1.0 / ah);
+                    float dv = ((float)uc[q][e] - (float)um) * (float)(dxi0)*rh;
+                    dv += ((float)vc[q][e] - (float)vm[q][e]) * (float)(dxi1)*rh;
+                    const float wk = (float)((double)wc[q][e] - mk);
+                    const float wkm = (float)((double)wm[q][e] - mkm);
+                    dv += (wk * (float)(1.0 / a0) - wkm * (float)(1.0 / a0m)) * (float)dxi2;
+                    d[e] = (TS)dv;
+                }
+                um = uc[q][e];
+                bufr[2 * ((i + e) * S + (rb >> 1)) + (rb & 1)] = d[e];
             }
-            if (div_out) div_out[oo[q]] = d;
-            bufr[2 * (i * S + (rb >> 1)) + (rb & 1)] = d;
+            if (div_out) *reinterpret_cast<VT *>(div_out + oo[q]) = d;
         }
     }
     __syncthreads();
@@ -302,8 +316,11 @@ __global__ __launch_bounds__(512) void div_fftx_kernel(Geo g, const TS *u, const
         }
         return;
     }
-    for (int q = threadIdx.x; q < nxh * S; q += blockDim.x) {
-        const int m = q % nxh, pb = q / nxh;
+    const int nxhalf = g.nx / 2;  // the last column after the others, which need no division
+    for (int q = threadIdx.x; q < (nxh << logS); q += blockDim.x) {
+        const bool last = q >= nxhalf << logS;
+        const int m = last ? nxhalf : q & (nxhalf - 1);
+        const int pb = last ? q - (nxhalf << logS) : q >> (logx - 1);
         const C2<TS> z = buf[m * S + pb];
         const C2<TS> zm = buf[((g.nx - m) & (g.nx - 1)) * S + pb];
         const C2<TS> xa{TS(0.5) * (z.x + zm.x), TS(0.5) * (z.y - zm.y)};
@@ -1134,13 +1151,18 @@ static int run_pressure(pycles_pressure_plan *P, const pycles_ref *ref, void *u,
     const int bx = S * g.nx / 8;
     const long long waves = (long long)(g.ny / (2 * S)) * g.nz * ((bx + 63) / 64);
     const int dbx = waves < 4096 && bx >= 32 && bx <= 128 ? 4 * bx : bx;
-#define DIV_FFTX(TR_)                                                                                          \
-    hipLaunchKernelGGL((div_fftx_kernel<TS, TR_>), dim3(g.ny / (2 * S), g.nz), dim3(dbx), rowsmem, st, g,       \
+    constexpr int V = 16 / sizeof(TS);
+    const bool wdiv = (((uintptr_t)u | (uintptr_t)v | (uintptr_t)w | (uintptr_t)div) & 15) == 0;
+#define DIV_FFTX(TR_, V_)                                                                                      \
+    hipLaunchKernelGGL((div_fftx_kernel<TS, TR_, V_>), dim3(g.ny / (2 * S), g.nz), dim3(dbx), rowsmem, st, g,       \
                        (const TS *)u, (const TS *)v, (const TS *)w, ref->alpha0, ref->alpha0_half, P->partial,  \
                        P->mean, cfl_out, (TS *)div, (C2<TS> *)P->spec, (const C2<TS> *)P->twx, P->logx, P->nxh, \
                        P->nxp, logS)
-    if (P->planes) DIV_FFTX(true);
-    else DIV_FFTX(false);
+    // the plane form's small grids have four cells per thread: single cells there
+    // (256 x 64 x 75 FP32, a projection and its RK3 stage: 73.5 us against 74.2)
+    if (P->planes) DIV_FFTX(true, 1);
+    else if (wdiv) DIV_FFTX(false, V);
+    else DIV_FFTX(false, 1);
 #undef DIV_FFTX
     PYCLES_CHECK_LAUNCH();
     if (P->planes) {
@@ -1184,7 +1206,6 @@ static int run_pressure(pycles_pressure_plan *P, const pycles_ref *ref, void *u,
 #undef IFFTX
     PYCLES_CHECK_LAUNCH();
     const ZSplit zs = correct_zsplit(g.plane, g.nz, g.gw);
-    constexpr int V = 16 / sizeof(TS);
     const bool wide = (((uintptr_t)u | (uintptr_t)v | (uintptr_t)w | (uintptr_t)p) & 15) == 0;
     const dim3 cgrid((unsigned)((g.plane / (wide ? V : 1) + 255) / 256), zs.nch);
     if (wide)

@@ -509,3 +509,32 @@ def test_fp32_advection_forms(n, orders, moist):
         err = np.abs(got - want).max()
         print(k, "error / bound", err / tol, flush=True)
         assert err <= tol, (k, err, tol)
+
+
+@pytest.mark.parametrize("n", [(8, 8, 5), (16, 64, 7), (64, 32, 9), (512, 64, 6), (2048, 16, 3), (256, 128, 70)])
+def test_fp32_projection_alignment(n):
+    """The FP32 projection by 16-byte accesses and, with the fields off a
+    16-byte boundary, by single ones: the same operations on the same values,
+    so the same bits."""
+    import torch
+    from pycles_amd import _capi
+    from pycles_amd import _device as D
+    nx, ny, nz = n
+    gw = 3
+    nzg, N = nz + 2 * gw, nx * ny * (nz + 2 * gw)
+    alpha = 0.8 + 0.5 * np.arange(nzg) / nzg
+    prof = {"rho0": 1.0 / alpha, "rho0_half": 1.0 / (alpha - 0.004), "alpha0": alpha, "alpha0_half": alpha - 0.004, "p0": alpha,
+            "p0_half": alpha}
+    dp = {k: _dev(v) for k, v in prof.items()}
+    ref = _capi.Ref(*[dp[k].data_ptr() for k in ("rho0", "rho0_half", "alpha0", "alpha0_half", "p0", "p0_half")])
+    f = _dev(np.random.default_rng(nx).standard_normal(3 * N).astype(np.float32))
+    plan = _capi.PressurePlan(_dims(n, gw, (50.0, 60.0, 20.0)), prof["rho0"].ctypes.data, prof["rho0_half"].ctypes.data, D.F32)
+    out = []
+    for shift in (0, 1):
+        buf = torch.zeros(5 * N + 4, dtype=torch.float32, device="cuda")
+        buf[shift:shift + 3 * N] = f
+        ptr = [buf.data_ptr() + 4 * (shift + q * N) for q in range(5)]
+        plan.update(ref, *ptr, 0.75, None, D.stream())
+        out.append(buf[shift:shift + 5 * N].cpu().numpy())
+    assert np.isfinite(out[0]).all() and np.abs(out[0][3 * N:]).max() > 0
+    assert np.array_equal(out[0], out[1])
