@@ -139,7 +139,7 @@ static inline long long advyz_blocks(int nx, int ny, int nz) {
 // 64 x 64 x 81 levels: 44 us with chunks of 21, 20 with 6; FP32 on 384 x 250 x
 // 106: 128 with 27, 124 with 14.
 static inline ZSplit thermo_zsplit(int nx, int ny, int nzg) {
-    const long long cols = (long long)((nx + 63) / 64) * ((ny + 3) / 4);
+    const long long cols = ((long long)nx * ny + 255) / 256;
     int want = 1;
     while (cols * want < 4096 && nzg / (want * 2) >= (cols * want < 512 ? 4 : cols * want < 2048 ? 8 : 16)) want *= 2;
     return zsplit_ceil(nzg, want);

@@ -190,9 +190,9 @@ extern "C" int pycles_thermo_sa(const pycles_dims *dims, const pycles_ref *ref, 
     const ZSplit zs = thermo_zsplit(g.nx, g.ny, g.nzg);
     a.kchunk = zs.len;
     const int nch = zs.nch;
-    dim3 blk(64, 4), grd((g.nx + 63) / 64, (g.ny + 3) / 4, nch);
     hipStream_t st = (hipStream_t)stream;
     if (precision == PYCLES_F64) {
+        const dim3 blk(64, 4), grd((g.nx + 63) / 64, (g.ny + 3) / 4, nch);
         const size_t smem = (size_t)(a.ntab + 3 * (a.kchunk + 2)) * sizeof(double);
         if (a.wt_over)
             hipLaunchKernelGGL(thermo_sa_f64_kernel<true>, grd, blk, smem, st, g, a);
@@ -200,7 +200,7 @@ extern "C" int pycles_thermo_sa(const pycles_dims *dims, const pycles_ref *ref, 
             hipLaunchKernelGGL(thermo_sa_f64_kernel<false>, grd, blk, smem, st, g, a);
     }
     else if (precision == PYCLES_F32)
-        return thermo_sa_f32_launch(g, a, grd, blk, st);
+        return thermo_sa_f32_launch(g, a, dim3((unsigned)((g.plane + 255) / 256), 1, nch), dim3(256), st);
     else {
         pycles_set_error("bad precision %d", precision);
         return PYCLES_ERR_ARG;
@@ -248,10 +248,8 @@ __global__ __launch_bounds__(256) void thermo_dry_kernel(Geo g, DryArgs a) {
         }
     }
     __syncthreads();
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int j = blockIdx.y * blockDim.y + threadIdx.y;
-    if (i >= g.nx || j >= g.ny) return;
-    const long long col = (long long)j * g.nx + i;
+    const long long col = (long long)blockIdx.x * 256 + tid;
+    if (col >= g.plane) return;
     const TS *s = (const TS *)a.s;
     TS *wt = (TS *)a.wt;
     TS *To = (TS *)a.T;
@@ -329,7 +327,7 @@ extern "C" int pycles_thermo_dry(const pycles_dims *dims, const pycles_ref *ref,
     if (zs.len > DRY_KMAX) zs = zsplit_ceil(g.nzg, (g.nzg + DRY_KMAX - 1) / DRY_KMAX);
     a.kchunk = zs.len;
     const int nch = zs.nch;
-    dim3 blk(64, 4), grd((g.nx + 63) / 64, (g.ny + 3) / 4, nch);
+    dim3 blk(256), grd((unsigned)((g.plane + 255) / 256), 1, nch);
     hipStream_t st = (hipStream_t)stream;
     if (precision == PYCLES_F64)
         launch_dry<double>(g, a, grd, blk, st);

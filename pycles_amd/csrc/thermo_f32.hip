@@ -63,11 +63,10 @@ __global__ __launch_bounds__(256, MLP ? 4 : 5) void thermo_sa_f32_kernel(Geo g, 
     if (tid < 4) cnt[tid] = 0;
     if (MLP) mlp::stage(a.mlp, &msm->w, tid, nthr);
     __syncthreads();
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int j = blockIdx.y * blockDim.y + threadIdx.y;
+    const long long lin = (long long)blockIdx.x * 256 + tid;
     unsigned ctr[4] = {0, 0, 0, 0};  // one thread's counts fit in 32 bits
-    const bool active = i < g.nx && j < g.ny;
-    const long long col = active ? (long long)j * g.nx + i : 0;
+    const bool active = lin < g.plane;
+    const long long col = active ? lin : 0;
     float *s = sreg((float *)a.s);
     float *qtp = sreg((float *)a.qt);
     float *wt = sreg((float *)a.wt);

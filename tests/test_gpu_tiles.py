@@ -538,3 +538,37 @@ def test_fp32_projection_alignment(n):
         out.append(buf[shift:shift + 5 * N].cpu().numpy())
     assert np.isfinite(out[0]).all() and np.abs(out[0][3 * N:]).max() > 0
     assert np.array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("n", [(17, 13, 9), (70, 9, 13), (24, 31, 40), (10, 25, 20)])
+@pytest.mark.parametrize("precision", ["f64", "f32"])
+def test_saturation_adjustment_columns(n, precision):
+    """Columns do not depend on the plane that holds them: the columns of a plane
+    that does not fill the kernels' blocks of 256, below and above one block,
+    give the bits that they give within a plane of whole blocks."""
+    import torch
+    from pycles_amd.Simulation3d import Simulation3d
+    from tests.helpers import host_case
+    from tests.test_gpu_parity import _saturating
+    nx, ny, nz = n
+    N = (128, 32)
+    state, out = None, []
+    for px, py in (N, (nx, ny)):
+        nl, Gr, RS, Th, fields = host_case(px, py, nz, seed=4)
+        nl["mi355x"]["precision"] = precision
+        fields = _saturating(Gr, fields)
+        sim = Simulation3d().initialize(nl, Gr=Gr, Ref=RS, Th=Th, fields=fields)
+        if state is None:
+            state = {k: (sim.PV.field(k).clone(), sim.PV.base.get(k)) for k in sim.PV.index_name}
+        else:
+            for k, (f, base) in state.items():
+                sim.PV.field(k).copy_(f[:, :ny, :nx])
+                if base is not None:
+                    sim.PV.base[k] = base
+        sim.Th.update(sim.Gr, sim.Ref, sim.PV, sim.DV, wt_overwrite=True)
+        out.append({k: sim.DV.field(k).clone() for k in ("temperature", "qv", "ql", "alpha", "buoyancy", "buoyancy_frequency")}
+                   | {"w": sim.PV.tend("w").clone(), "qt": sim.PV.field("qt").clone()})
+    torch.cuda.synchronize()
+    assert float((out[1]["ql"] > 0).double().mean()) > 0.05
+    for k, a in out[1].items():
+        assert torch.equal(a, out[0][k][:, :ny, :nx].contiguous()), k
