@@ -117,7 +117,8 @@ int pycles_advection(const pycles_dims *dims, const pycles_ref *ref, const void 
  * the caller keeps that stage's input unchanged and passes it as the copy of
  * stages 1 and 2; at rk_step 2 out_* may be that same array (each cell's copy
  * is read before its output is written).  The tendency arrays keep the x and
- * y contributions.
+ * y contributions (in FP32, where the y and z passes run as one kernel, the x
+ * contribution).
  * Same bits as pycles_advection then pycles_rk3_stage.  Needs the momentum. */
 int pycles_advection_rk3(const pycles_dims *dims, const pycles_ref *ref, const void *const vel[3],
                          void *const tend_vel[3], int nscal, const void *const *scal,

@@ -104,6 +104,9 @@ struct PolicyF64 {
     // 17, 64^3 23.5 against 12 + 13, and a launch less.
     static constexpr bool kFuseYZ = false;
     static constexpr int kYZWaves = 1;
+    // the fused kernel's RK3 forms store the tendencies with the y contribution
+    // too, as the y pass does
+    static constexpr bool kYZTend = true;
     // waves per SIMD the z pass is held to (<= 168 VGPRs): its stage-2 form
     // otherwise takes 171 and runs 2 waves
     static constexpr int kZWaves = 3;
@@ -189,6 +192,7 @@ struct PolicyF32 {
     using SFlux = SF32;
     static constexpr bool kBase = true;
     static constexpr bool kFuseYZ = true;  // y and z passes fused (WENO5)
+    static constexpr bool kYZTend = false;  // whose RK3 forms leave the tendencies with the x contribution
     static constexpr int kYZWaves = 3;     // waves per SIMD of the fused pass (its LDS allows 3 blocks per CU)
     static constexpr int kZWaves = 1;      // the z pass's registers as the compiler allocates them
     static constexpr bool kXVec = false;   // the x pass stays the row-staged kernel
@@ -778,9 +782,10 @@ __global__ __launch_bounds__(256) void adv_y(Geo g, Prof pr, Fields fl, int jchu
 //  C. (barrier) each cell's tendency takes the y flux difference (the lower
 //     face from LDS), rounded as the y pass stores it, then the z flux
 //     difference, in the per-variable order of the separate passes, so the
-//     bits are theirs; then the RK3 stage as in the z pass.
+//     bits are theirs; then the RK3 stage as in the z pass, which in FP64
+//     leaves the tendencies as the y pass does (P::kYZTend).
 // Against the y pass followed by the z pass this drops the y pass's tendency
-// read and write and its re-read of the fields.  Columns beyond a partial
+// read and (but for FP64's RK3 stages) write and its re-read of the fields.  Columns beyond a partial
 // tile (nx not a multiple of 64, ny of TY; PART) march wrapped copies of
 // real columns and store nothing, so every thread reaches every barrier.
 // A chunk holds at most ADV_YZ_KMAX levels (advyz_zsplit): its level
@@ -1040,20 +1045,25 @@ __global__ __launch_bounds__(64 * TY, P::kYZWaves) void adv_yz(Geo g, Prof pr, F
         if constexpr (!FIRST) {
             // C: y then z flux differences, then the stage update
             const double ah = prof(3, c), a0 = prof(2, c);
-            TS tn[5] = {};
+            TS t1[5] = {}, tn[5] = {};
 #pragma unroll
             for (int sc = 0; sc < NSC; ++sc) {
                 const double brho = P::kBase ? prof((4 + sc) % NPR, c) * rh : 0.0;
-                const TS t1 = told[sc] - P::x_scal_div(Fy[sc], flx[b][sc][ty][tx], Vc, Vp, ah, dyi, brho);
-                tn[sc] = add_rn(t1, -P::template scal_div<true>(Fs[sc], Fs_prev[sc], ah, dzi, 1.0));
+                t1[sc] = told[sc] - P::x_scal_div(Fy[sc], flx[b][sc][ty][tx], Vc, Vp, ah, dyi, brho);
+                tn[sc] = add_rn(t1[sc], -P::template scal_div<true>(Fs[sc], Fs_prev[sc], ah, dzi, 1.0));
             }
-            const TS tu = (TS)(told[VU] - P::mom_div(Fy[FU], flx[b][FU][ty][tx], ah, dyi));
-            const TS tv = (TS)(told[VV] - P::mom_div(Fy[FV], flx[b][FV][ty][tx], ah, dyi));
-            const TS tw = (TS)(told[VW] - P::mom_div(Fy[FW], flx[b][FW][ty][tx], a0, dyi));
-            tn[VU] = add_rn(tu, -P::mom_div(Fu, Fu_prev, ah, dzi));
-            tn[VV] = add_rn(tv, -P::mom_div(Fv, Fv_prev, ah, dzi));
-            tn[VW] = add_rn(tw, -P::mom_div(Fw, Fw_prev, a0, dzi));
+            t1[VU] = (TS)(told[VU] - P::mom_div(Fy[FU], flx[b][FU][ty][tx], ah, dyi));
+            t1[VV] = (TS)(told[VV] - P::mom_div(Fy[FV], flx[b][FV][ty][tx], ah, dyi));
+            t1[VW] = (TS)(told[VW] - P::mom_div(Fy[FW], flx[b][FW][ty][tx], a0, dyi));
+            tn[VU] = add_rn(t1[VU], -P::mom_div(Fu, Fu_prev, ah, dzi));
+            tn[VV] = add_rn(t1[VV], -P::mom_div(Fv, Fv_prev, ah, dzi));
+            tn[VW] = add_rn(t1[VW], -P::mom_div(Fw, Fw_prev, a0, dzi));
             if (own) {
+                if (RKM != 0 && P::kYZTend) {
+#pragma unroll
+                    for (int v = 0; v < 5; ++v)
+                        if (v < NSC || v >= VU) sts_((TS *)fl.t[v], o, t1[v]);
+                }
                 if (RKM == 0) {
 #pragma unroll
                     for (int v = 0; v < 5; ++v)
