@@ -278,6 +278,16 @@ int pycles_pressure_plan_create(const pycles_dims *dims, const double *rho0_host
                                 const double *rho0_half_host, int precision,
                                 pycles_pressure_plan **plan);
 void pycles_pressure_plan_destroy(pycles_pressure_plan *plan);
+/* The form of the z solve that a plan of these sizes takes (a host rule, no
+ * device call; negative: the error plan_create returns): general (one thread
+ * per column, any size), columns (stored pivots, 16 columns of all levels in
+ * LDS), planes (y transforms and solve of one kx in one kernel), planes with
+ * their pivots staged in LDS.  The results agree to rounding. */
+#define PYCLES_PRESSURE_GENERAL 0
+#define PYCLES_PRESSURE_COLUMNS 1
+#define PYCLES_PRESSURE_PLANES 2
+#define PYCLES_PRESSURE_PLANES_STAGED 3
+int pycles_pressure_form(const pycles_dims *dims, int precision);
 /* Replaces PressureSolver.update (PressureSolver.pyx:38-81): remove the
  * level mean of w, divergence of rho0*u, horizontal real FFT, per-wavenumber
  * tridiagonal solve in z with the (0,0) mode set to zero, inverse FFT,

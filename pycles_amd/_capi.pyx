@@ -122,6 +122,7 @@ cdef extern from "pycles_amd.h":
                                     const double *rho0_half_host, int precision,
                                     pycles_pressure_plan **plan)
     void pycles_pressure_plan_destroy(pycles_pressure_plan *plan)
+    int pycles_pressure_form(const pycles_dims *dims, int precision)
     int pycles_pressure_update(pycles_pressure_plan *plan, const pycles_ref *ref, void *u, void *v,
                                void *w, void *p, void *div, double dt, double *cfl_out, void *stream)
     int pycles_divergence(const pycles_dims *dims, const pycles_ref *ref, const void *u,
@@ -241,6 +242,13 @@ cdef class SAOptions:
         self.o.counters = <long long *> _p(counters)
         self.o.wt_overwrite = 1 if wt_overwrite else 0
         self.o.secant_tol = secant_tol
+
+
+def pressure_form(Dims dims, int precision):
+    """0 general, 1 columns, 2 planes, 3 planes with staged pivots."""
+    cdef int form = pycles_pressure_form(&dims.d, precision)
+    _check(min(form, 0))
+    return form
 
 
 cdef class PressurePlan:

@@ -949,17 +949,41 @@ __global__ void divergence_kernel(Geo g, const TS *u, const TS *v, const TS *w, 
 }
 
 // ---------------------------------------------------------------------------
-extern "C" int pycles_pressure_plan_create(const pycles_dims *dims, const double *rho0, const double *rho0_half,
-                                           int precision, pycles_pressure_plan **out) {
+// The form of a plan's z solve (PYCLES_PRESSURE_*) and the LDS of its blocks.
+// The plane form where its blocks are all resident at once and either half the
+// CUs have one or a plane is little work for the others to wait for: 256 x 256
+// x 60 FP32 174 -> 162 us a projection, 64 x 64 x 64 FP64 gains 10 us, 64 x 128 x
+// 70 (33 blocks of 8960 values) would lose 20; with staged pivots, or else
+// without.  Then stored pivots for few columns, their blocks all resident at once.
+static int pressure_form(const Geo &g, int precision, size_t *lds) {
+    const bool f64 = precision == PYCLES_F64;
+    const int nxh = g.nx / 2 + 1;
+    const long long cu = 160 * 1024;  // LDS of a CU
+    if (nxh >= 128 || (long long)g.ny * g.nz <= 5120) {
+        *lds = f64 ? plane_lds_bytes<double, true>(g.ny, g.nz) : plane_lds_bytes<float, true>(g.ny, g.nz);
+        if ((long long)*lds <= cu && nxh <= 256 * (cu / (long long)*lds)) return PYCLES_PRESSURE_PLANES_STAGED;
+        *lds = f64 ? plane_lds_bytes<double, false>(g.ny, g.nz) : plane_lds_bytes<float, false>(g.ny, g.nz);
+        if ((long long)*lds <= cu && nxh <= 256 * (cu / (long long)*lds)) return PYCLES_PRESSURE_PLANES;
+    }
+    *lds = f64 ? thomas_lds_bytes<double>(g.nz) : thomas_lds_bytes<float>(g.nz);
+    const long long blocks = ((long long)g.ny * nxh + TL_COLS - 1) / TL_COLS;
+    if ((long long)*lds <= cu && blocks <= 256 * (cu / (long long)*lds) && blocks <= 2048) return PYCLES_PRESSURE_COLUMNS;
+    *lds = 0;
+    return PYCLES_PRESSURE_GENERAL;
+}
+
+// Whether a plan can be made for these sizes, and their logarithms
+static int pressure_check(const pycles_dims *dims, int precision, int *logx, int *logy) {
     int rc = pycles_check_dims(dims);
     if (rc) return rc;
-    if (!out || !rho0 || !rho0_half || (precision != PYCLES_F64 && precision != PYCLES_F32)) {
-        pycles_set_error("pressure_plan_create: bad arguments");
+    if (precision != PYCLES_F64 && precision != PYCLES_F32) {
+        pycles_set_error("pressure: bad precision %d", precision);
         return PYCLES_ERR_ARG;
     }
-    Geo g = make_geo(dims);
-    const int logx = ilog2(g.nx), logy = ilog2(g.ny);
-    if (logx < 3 || logy < 3 || g.nx > 4096 || g.ny > 4096) {
+    const Geo g = make_geo(dims);
+    *logx = ilog2(g.nx);
+    *logy = ilog2(g.ny);
+    if (*logx < 3 || *logy < 3 || g.nx > 4096 || g.ny > 4096) {
         pycles_set_error("pressure: nx, ny must be powers of two in [8, 4096] (got %d, %d)", g.nx, g.ny);
         return PYCLES_ERR_UNSUPPORTED;
     }
@@ -967,6 +991,27 @@ extern "C" int pycles_pressure_plan_create(const pycles_dims *dims, const double
         pycles_set_error("pressure: nz must be in [2, %d] (got %d)", PRESSURE_MAX_NZ, g.nz);
         return PYCLES_ERR_UNSUPPORTED;
     }
+    return PYCLES_OK;
+}
+
+extern "C" int pycles_pressure_form(const pycles_dims *dims, int precision) {
+    int logx, logy;
+    const int rc = pressure_check(dims, precision, &logx, &logy);
+    if (rc) return rc;
+    size_t lds;
+    return pressure_form(make_geo(dims), precision, &lds);
+}
+
+extern "C" int pycles_pressure_plan_create(const pycles_dims *dims, const double *rho0, const double *rho0_half,
+                                           int precision, pycles_pressure_plan **out) {
+    if (!out || !rho0 || !rho0_half) {
+        pycles_set_error("pressure_plan_create: bad arguments");
+        return PYCLES_ERR_ARG;
+    }
+    int logx, logy;
+    const int rc = pressure_check(dims, precision, &logx, &logy);
+    if (rc) return rc;
+    const Geo g = make_geo(dims);
     pycles_pressure_plan *P = new pycles_pressure_plan();
     memset(P, 0, sizeof(*P));
     P->g = g;
@@ -1027,37 +1072,22 @@ extern "C" int pycles_pressure_plan_create(const pycles_dims *dims, const double
         }                                                   \
     } while (0)
     ALLOC(P->spec, nspec * cs);
-    // the z solve's form for few columns: its blocks all resident at once
     {
-        const size_t lds = precision == PYCLES_F64 ? thomas_lds_bytes<double>(g.nz) : thomas_lds_bytes<float>(g.nz);
-        const long long blocks = ((long long)g.ny * P->nxh + TL_COLS - 1) / TL_COLS;
-        P->thomas_lds = lds <= 160 * 1024 && blocks <= 256 * (long long)(160 * 1024 / lds) && blocks <= 2048;
-        if (P->thomas_lds && lds > 64 * 1024) {
-            const void *fn = precision == PYCLES_F64 ? (const void *)thomas_lds_kernel<double>
-                                                     : (const void *)thomas_lds_kernel<float>;
-            // the limit for every plan of this form, not this one's size
-            if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess)
-                P->thomas_lds = false;
+        // the LDS limit is raised for every plan of the form, not to this one's size
+        size_t lds;
+        int form = pressure_form(g, precision, &lds);
+        const bool f64 = precision == PYCLES_F64;
+        const void *fn = form == PYCLES_PRESSURE_COLUMNS ? (f64 ? (const void *)thomas_lds_kernel<double> : (const void *)thomas_lds_kernel<float>)
+                       : form == PYCLES_PRESSURE_PLANES ? (f64 ? (const void *)plane_solve_kernel<double, false> : (const void *)plane_solve_kernel<float, false>)
+                                                        : (f64 ? (const void *)plane_solve_kernel<double, true> : (const void *)plane_solve_kernel<float, true>);
+        if (form != PYCLES_PRESSURE_GENERAL && lds > 64 * 1024 &&
+            hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess) {
+            (void)hipGetLastError();
+            form = PYCLES_PRESSURE_GENERAL;
         }
-        // the plane form where its blocks are all resident at once and either
-        // half the CUs have one or a plane is little work for the others to
-        // wait for: 256 x 256 x 60 FP32 174 -> 162 us a projection, 64 x 64 x 64
-        // FP64 gains 10 us, 64 x 128 x 70 (33 blocks of 8960 values) would lose 20;
-        // with staged pivots, or else without
-        const bool few = P->nxh >= 128 || (long long)g.ny * nz <= 5120;
-        for (int stg = 1; few && stg >= 0 && !P->planes; --stg) {
-            const size_t pl = precision == PYCLES_F64
-                                  ? (stg ? plane_lds_bytes<double, true>(g.ny, nz) : plane_lds_bytes<double, false>(g.ny, nz))
-                                  : (stg ? plane_lds_bytes<float, true>(g.ny, nz) : plane_lds_bytes<float, false>(g.ny, nz));
-            if (pl > 160 * 1024 || P->nxh > 256 * (int)(160 * 1024 / pl)) continue;
-            P->planes = 1 + stg;
-            P->plane_lds = pl;
-            const void *fn = precision == PYCLES_F64
-                                 ? (stg ? (const void *)plane_solve_kernel<double, true> : (const void *)plane_solve_kernel<double, false>)
-                                 : (stg ? (const void *)plane_solve_kernel<float, true> : (const void *)plane_solve_kernel<float, false>);
-            if (pl > 64 * 1024 && hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess)
-                P->planes = 0;
-        }
+        P->thomas_lds = form == PYCLES_PRESSURE_COLUMNS;
+        P->planes = form == PYCLES_PRESSURE_PLANES ? 1 : form == PYCLES_PRESSURE_PLANES_STAGED ? 2 : 0;
+        P->plane_lds = lds;
         if (P->planes || P->thomas_lds) {
             ALLOC(P->pm, sizeof(double) * (size_t)g.nz * g.ny * P->nxh);
             ALLOC(P->pc, es * (size_t)g.nz * g.ny * P->nxh);

@@ -152,3 +152,18 @@ def test_advection_z_chunks_fit_their_lds_rows(lib):
             for kern, cap in ((2, 128), (4, 96)):
                 nch, ln = _chunks(lib, kern, plane + (nz,))
                 assert ln <= cap and nch * ln >= nz and (nch - 1) * ln < nz, (kern, plane, nz, nch, ln)
+
+
+def test_pressure_forms_of_the_operator_tests(lib):
+    """The form of the projection's z solve at the sizes that hold each form to
+    the oracle (test_gpu_routes.py, test_gpu_parity.py, test_gpu_tiles.py):
+    0 general, 1 stored pivots for few columns, 2 planes, 3 planes with staged
+    pivots; and the refusals of the plan."""
+    form = lambda n, prec, gw=3: lib.pycles_pressure_form(C.byref(_dims(n=n, gw=gw)), prec)  # noqa: E731
+    for n, f64, f32 in (((16, 32, 315), 1, 1), ((16, 32, 317), 0, 1), ((16, 32, 499), 0, 1), ((16, 32, 501), 0, 0),
+                        ((64, 128, 41), 1, 1), ((64, 64, 100), 1, 1), ((32, 32, 250), 1, 1), ((128, 256, 131), 0, 0),
+                        ((256, 128, 83), 0, 2), ((256, 64, 160), 0, 2), ((64, 64, 80), 2, 3), ((64, 64, 81), 1, 1),
+                        ((16, 8, 316), 3, 3), ((256, 64, 75), 3, 3), ((256, 128, 70), 2, 2), ((512, 512, 256), 0, 0)):
+        assert (form(n, 0), form(n, 1)) == (f64, f32), n
+    assert form((12, 16, 8), 0) == -3 and form((16, 16, 2049), 1) == -3
+    assert form((16, 16, 8), 7) == -1 and form((16, 16, 8), 0, gw=9) == -1
