@@ -950,16 +950,30 @@ __global__ void divergence_kernel(Geo g, const TS *u, const TS *v, const TS *w, 
 
 // ---------------------------------------------------------------------------
 // The form of a plan's z solve (PYCLES_PRESSURE_*) and the LDS of its blocks.
-// The plane form where its blocks are all resident at once and either half the
-// CUs have one or a plane is little work for the others to wait for: 256 x 256
-// x 60 FP32 174 -> 162 us a projection, 64 x 64 x 64 FP64 gains 10 us, 64 x 128 x
-// 70 (33 blocks of 8960 values) would lose 20; with staged pivots, or else
-// without.  Then stored pivots for few columns, their blocks all resident at once.
+// The plane form where its blocks are all resident at once (with staged pivots,
+// or else without) and, by the us of a projection with it and without:
+// - fewer blocks than half the CUs: a plane of at most 5120 values.  64 x 64 x 75
+//   FP64 49 and 53, 64 x 128 x 40 48 and 49, x 50 55 and 53, x 70 81 and 59;
+// - a block per CU at most: any plane that fits.  256 x 64 x 75 FP32 57 and 62, 256 x
+//   256 x 60 104 and 116, FP64 164 and 165;
+// - more: the other kernels fill the chip too, and read and write the spectrum
+//   as fast once it is large.  At most 2^17 columns and 2^21 cells (FP32 rows
+//   of 1024 or more: 3 2^19), or 2^14 columns of any depth.  512 x 128 x 25 FP64 91
+//   and 99, x 38 123 and 116; 512 x 32 x 150 138 and 146; 2048 x 64 x 20 141 and 125;
+//   1024 x 64 x 20 FP32 60 and 62, x 30 86 and 80; 1024 x 128 x 40 161 and 127.
+// Then stored pivots for few columns, their blocks all resident at once.
+static bool planes_pay(const Geo &g, bool f64) {
+    const int nxh = g.nx / 2 + 1;
+    if (nxh < 128) return (long long)g.ny * g.nz <= 5120;
+    if (nxh <= 256) return true;
+    return g.plane <= 1 << 17 &&
+           (g.plane <= 1 << 14 || g.plane * g.nz <= (!f64 && g.nx >= 1024 ? 3 << 19 : 1 << 21));
+}
 static int pressure_form(const Geo &g, int precision, size_t *lds) {
     const bool f64 = precision == PYCLES_F64;
     const int nxh = g.nx / 2 + 1;
     const long long cu = 160 * 1024;  // LDS of a CU
-    if (nxh >= 128 || (long long)g.ny * g.nz <= 5120) {
+    if (planes_pay(g, f64)) {
         *lds = f64 ? plane_lds_bytes<double, true>(g.ny, g.nz) : plane_lds_bytes<float, true>(g.ny, g.nz);
         if ((long long)*lds <= cu && nxh <= 256 * (cu / (long long)*lds)) return PYCLES_PRESSURE_PLANES_STAGED;
         *lds = f64 ? plane_lds_bytes<double, false>(g.ny, g.nz) : plane_lds_bytes<float, false>(g.ny, g.nz);

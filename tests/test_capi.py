@@ -167,3 +167,15 @@ def test_pressure_forms_of_the_operator_tests(lib):
         assert (form(n, 0), form(n, 1)) == (f64, f32), n
     assert form((12, 16, 8), 0) == -3 and form((16, 16, 2049), 1) == -3
     assert form((16, 16, 8), 7) == -1 and form((16, 16, 8), 0, gw=9) == -1
+
+
+def test_pressure_planes_stop_where_they_are_slower(lib):
+    """Plans of more planes than CUs: the plane form up to the sizes where it
+    was measured as fast as the other kernels, not beyond."""
+    form = lambda n, prec: lib.pycles_pressure_form(C.byref(_dims(n=n)), prec)  # noqa: E731
+    for n in ((2048, 64, 20), (1024, 128, 20), (1024, 256, 7), (512, 1024, 3), (512, 256, 17), (4096, 64, 8), (4096, 8, 80)):
+        assert 0 <= form(n, 0) < 2 and 0 <= form(n, 1) < 2, n
+    for n in ((1024, 128, 40), (1024, 64, 30), (2048, 32, 31)):
+        assert 0 <= form(n, 1) < 2, n
+    for n in ((512, 64, 64), (512, 256, 15), (512, 32, 128), (1024, 64, 20), (1024, 16, 128), (2048, 16, 40), (4096, 8, 40)):
+        assert form(n, 0) >= 2 and form(n, 1) >= 2, n
