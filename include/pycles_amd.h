@@ -106,6 +106,10 @@ int pycles_advection(const pycles_dims *dims, const pycles_ref *ref, const void 
                      void *const tend_vel[3], int nscal, const void *const *scal,
                      void *const *tend_scal, const pycles_scalar_base *base, int scalar_order,
                      int momentum_order, int precision, int flags, void *stream);
+/* Whether a call of these sizes runs its y and z passes as one kernel by
+ * default (1, else 0; a host rule, no device call; negative: an error). */
+int pycles_advection_yz_fused(const pycles_dims *dims, int nscal, int momentum, int scalar_order,
+                              int momentum_order, int precision);
 /* pycles_advection followed by the RK3 stage in the same sweep: TimeStepping.
  * update_third (TimeStepping.pyx:131-151) and the z boundary fill of
  * PrognosticVariables.update_all_bcs (PrognosticVariables.pyx:183-233;

@@ -77,9 +77,9 @@ class MomentumAdvection:
 
 def yz_fused(SA: ScalarAdvection, MA: MomentumAdvection, PV) -> bool:
     """Whether one call's y and z passes run as one fused kernel (the
-    library does so for FP32 storage, WENO5 scalars and momentum, with at
-    least one scalar); otherwise they are two kernels."""
-    return PV.precision == D.F32 and SA.order == 5 and MA.order == 5 and bool(_scalar_names(PV))
+    library's rule: WENO5 scalars and momentum with at least one scalar, in
+    FP32 storage, or in FP64 on small grids); otherwise they are two kernels."""
+    return _capi.advection_yz_fused(SA.dims, len(_scalar_names(PV)), True, SA.order, MA.order, PV.precision)
 
 
 def advect_rk3(SA: ScalarAdvection, MA: MomentumAdvection, TS, Gr, RS, PV, tend_zero=False, passes=0,

@@ -64,6 +64,8 @@ cdef extern from "pycles_amd.h":
                          void *const *tend_vel, int nscal, const void *const *scal,
                          void *const *tend_scal, const pycles_scalar_base *base, int scalar_order,
                          int momentum_order, int precision, int flags, void *stream)
+    int pycles_advection_yz_fused(const pycles_dims *dims, int nscal, int momentum, int scalar_order,
+                                  int momentum_order, int precision)
     int pycles_advection_rk3(const pycles_dims *dims, const pycles_ref *ref, const void *const *vel,
                              void *const *tend_vel, int nscal, const void *const *scal,
                              void *const *tend_scal, const pycles_scalar_base *base, int scalar_order,
@@ -288,6 +290,12 @@ def advection(Dims dims, Ref ref, vel, tend_vel, scal, tend_scal, ScalarBase bas
     _check(pycles_advection(&dims.d, &ref.r, v3, t3 if tend_vel is not None else NULL, ns, sc, ts,
                             &base.b if base is not None else NULL, scalar_order, momentum_order,
                             precision, flags, _p(stream)))
+
+
+def advection_yz_fused(Dims dims, int nscal, momentum, int scalar_order, int momentum_order, int precision):
+    cdef int r = pycles_advection_yz_fused(&dims.d, nscal, 1 if momentum else 0, scalar_order, momentum_order, precision)
+    _check(min(r, 0))
+    return r == 1
 
 
 def advection_rk3(Dims dims, Ref ref, vel, tend_vel, scal, tend_scal, ScalarBase base, int scalar_order,

@@ -143,3 +143,16 @@ extern "C" int pycles_advection_rk3(const pycles_dims *dims, const pycles_ref *r
     return advection_run(dims, ref, vel, tend_vel, nscal, scal, tend_scal, base, scalar_order, momentum_order,
                          precision, flags, &rk, stream);
 }
+
+extern "C" int pycles_advection_yz_fused(const pycles_dims *dims, int nscal, int momentum, int scalar_order,
+                                         int momentum_order, int precision) {
+    int rc = pycles_check_dims(dims);
+    if (rc) return rc;
+    if (precision != PYCLES_F64 && precision != PYCLES_F32) {
+        pycles_set_error("bad precision %d", precision);
+        return PYCLES_ERR_ARG;
+    }
+    const Geo g = make_geo(dims);
+    return scalar_order == 5 && momentum_order == 5 && momentum && nscal >= 1 &&
+           advyz_fused(precision == PYCLES_F32, g.nx, g.ny, g.nz);
+}

@@ -1566,7 +1566,7 @@ int launch(const Geo &g, const Prof &pr, const Fields &fl, hipStream_t st) {
     }
     // y and z fused (WENO5 with momentum and scalars), z-chunked like the z pass
     if constexpr (SO == 5 && MO == 5 && MOM && NSC >= 1) {
-        if ((fl.passes & 6) == 6 && (P::kFuseYZ || fl.fuse_yz || advyz_blocks(g.nx, g.ny, g.nz) <= 256)) {
+        if ((fl.passes & 6) == 6 && (fl.fuse_yz || advyz_fused(P::kFuseYZ, g.nx, g.ny, g.nz))) {
             // 4 rows per block: 8 rows halve the lower faces' extra work but
             // need more registers than 4 waves per SIMD allow with the RK3
             // stage (spills), and at 3 waves a 512-thread block fits once per CU

@@ -130,6 +130,13 @@ static inline ZSplit advyz_zsplit(int nx, int ny, int nz) {
 static inline long long advyz_blocks(int nx, int ny, int nz) {
     return (long long)((nx + 63) / 64) * ((ny + 3) / 4) * advyz_zsplit(nx, ny, nz).nch;
 }
+// Whether a WENO5 call with momentum and scalars takes it: in FP32 on any grid,
+// in FP64, where a CU holds one of its blocks, on grids of no more blocks than
+// CUs.  The count is that of the split above, made for 768 resident blocks:
+// 64 x 64 planes of 64 and 75 levels (256 and 240 blocks) are fused; 76 levels
+// (19 chunks of 4, 304 blocks) run the two passes, though 16 chunks of 5 would
+// be 256.
+static inline bool advyz_fused(bool f32, int nx, int ny, int nz) { return f32 || advyz_blocks(nx, ny, nz) <= 256; }
 // The thermodynamics kernels' chunks of the nzg ghosted levels (their LDS
 // holds len + 2 levels, so no chunk is longer than len): up to 4096 blocks.
 // Each chunk evaluates up to two levels of its neighbours, so chunks hold at

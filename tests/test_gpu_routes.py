@@ -8,15 +8,17 @@ from tests.helpers import host_case, oracle_sim
 pytestmark = pytest.mark.gpu
 
 
-def _sim(n, precision="f64", seed=21):
-    """A simulation of n cells with a divergence-free swirl and its fields."""
+def _sim(n, precision="f64", seed=21, swirl=True):
+    """A simulation of n cells, for operators with winds of both signs everywhere
+    (swirl; no state to step), and its fields."""
     import json
 
     from tests.test_gpu_parity import _gpu_sim, _swirl
     nl, Gr, RS, Th, fields = host_case(*n, seed=seed)
     nl = json.loads(json.dumps(nl))
     nl["mi355x"]["precision"] = precision
-    fields = _swirl(Gr, fields)
+    if swirl:
+        fields = _swirl(Gr, fields)
     return _gpu_sim(nl, Gr, RS, Th, fields), Gr, RS, Th, fields
 
 
@@ -132,3 +134,34 @@ def test_projection_form_against_the_oracle(gpu, n, precision, form):
         err = np.abs(a.astype(np.float64) - b).max() / np.abs(b).max()
         print(name, err, flush=True)
         assert err <= tol[q], (name, err)
+
+
+@pytest.mark.parametrize("n,fused", [((64, 64, 64), True), ((64, 64, 76), False)])
+def test_yz_switch(gpu, n, fused):
+    """On both sides of the FP64 switch (256 and 304 blocks) the default call
+    gives the bits of the passes launched one by one, and a timed step brackets
+    the passes that the untimed one runs, with its bits."""
+    import torch
+    from pycles_amd import _capi
+    from pycles_amd.Advection import advect_fused, yz_fused
+    sim = _sim(n)[0]
+    PV = sim.PV
+    assert yz_fused(sim.SA, sim.MA, PV) == fused
+    out = []
+    for seq in ((0,), (_capi.ADV_PASS_X, _capi.ADV_PASS_Y, _capi.ADV_PASS_Z)):
+        PV.zero_tendencies()
+        for p in seq:
+            advect_fused(sim.SA, sim.MA, sim.Gr, sim.Ref, PV, passes=p)
+        out.append(PV.tendencies.clone())
+    assert torch.equal(out[0], out[1])
+    steps = []
+    for timed in (False, True):
+        s = _sim(n, swirl=False)[0]
+        s.begin_run()
+        s.timers = [] if timed else None
+        s.step()
+        torch.cuda.synchronize()
+        steps.append((s.PV.values.clone(), s.PV.tendencies.clone()))
+    names = {a for a, _ in s.timers}
+    assert ("adv_yz_rk3" in names, "adv_z_rk3" in names) == (fused, not fused)
+    assert torch.equal(steps[0][0], steps[1][0]) and torch.equal(steps[0][1], steps[1][1])

@@ -177,3 +177,27 @@ def test_residual_check_logarithm_method():
     m = math.sqrt(2.0) - 1e-12
     t = (m - 1.0) / (m + 1.0)
     assert t ** 19 / 19 * 2 < 1e-15 < t ** 17 / 17 * 2
+
+
+def test_timed_passes_are_the_kernels_of_the_untimed_call():
+    """yz_fused, by which a timed stage picks the passes it brackets, is the
+    library's own rule: FP32 always, FP64 on grids of at most 256 blocks, WENO5
+    with a scalar only."""
+    from types import SimpleNamespace as N
+
+    from pycles_amd import _capi
+    from pycles_amd.Advection import yz_fused
+
+    def fused(n, precision, orders=(5, 5), scalars=("s",)):
+        names = ["u", "v", "w", *scalars]
+        PV = N(precision=precision, index_name=names, var_type=[0, 0, 0] + [1] * len(scalars))
+        return yz_fused(N(dims=_capi.Dims(n, 5, (50.0, 50.0, 20.0)), order=orders[0]), N(order=orders[1]), PV)
+
+    for n, small in (((64, 64, 64), True), ((64, 64, 75), True), ((24, 20, 16), True), ((64, 64, 76), False),
+                     ((128, 128, 64), False), ((512, 512, 256), False)):
+        nch, _ = _capi.launch_chunks(4, _capi.Dims(n, 5, (50.0, 50.0, 20.0)))
+        assert ((n[0] + 63) // 64 * ((n[1] + 3) // 4) * nch <= 256) == small
+        assert fused(n, _capi.F64) == small and fused(n, _capi.F32)
+    for orders in ((7, 7), (9, 5), (9, 9)):
+        assert not fused((64, 64, 64), _capi.F32, orders) and not fused((64, 64, 64), _capi.F64, orders)
+    assert not fused((64, 64, 64), _capi.F32, scalars=())
