@@ -136,6 +136,25 @@ def test_projection_form_against_the_oracle(gpu, n, precision, form):
         assert err <= tol[q], (name, err)
 
 
+def test_separate_passes_against_the_oracle(gpu):
+    """The x, y and z passes of moist WENO5 launched one by one (FP64, partial
+    tiles in every direction): the oracle's bits."""
+    import torch
+    from pycles_amd import _capi
+    from pycles_amd.Advection import advect_fused
+    sim, Gr, RS, Th, fields = _sim((24, 20, 16), seed=7)
+    for p in (_capi.ADV_PASS_X, _capi.ADV_PASS_Y, _capi.ADV_PASS_Z):
+        advect_fused(sim.SA, sim.MA, sim.Gr, sim.Ref, sim.PV, passes=p)
+    torch.cuda.synchronize()
+    osim = oracle_sim(Gr, RS, Th, fields, True)
+    osim.scalar_advection_update()
+    osim.momentum_advection_update()
+    gw = Gr.dims.gw
+    for n in ("u", "v", "w", "s", "qt"):
+        g = sim.PV.get_tendency_array(n, Gr)[gw:-gw, gw:-gw, gw:-gw]
+        assert np.array_equal(g, osim.pt(n)[gw:-gw, gw:-gw, gw:-gw]), n
+
+
 @pytest.mark.parametrize("n,fused", [((64, 64, 64), True), ((64, 64, 76), False)])
 def test_yz_switch(gpu, n, fused):
     """On both sides of the FP64 switch (256 and 304 blocks) the default call
