@@ -83,13 +83,6 @@ __device__ __forceinline__ void sts_(T *p, unsigned idx, T v) {
     __builtin_nontemporal_store(v, at(p, idx));
 }
 
-// tend -= d, or tend = 0 - d when the tendency is known to be zero (same bits).
-template <typename TS>
-__device__ __forceinline__ void sub_into(TS *p, unsigned o, TS d, bool zero) {
-    if (zero) *at(p, o) = TS(0) - d;
-    else *at(p, o) -= d;
-}
-
 // -------------------------------------------------------------------------
 // FP64 policy: storage and arithmetic in double, reference operation order.
 struct PolicyF64 {

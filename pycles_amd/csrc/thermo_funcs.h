@@ -65,12 +65,6 @@ template <class D = DivIeee> __device__ __forceinline__ double alpha_c(double p0
 template <class D = DivIeee> __device__ __forceinline__ double buoyancy_c(double alpha0, double alpha) {
     return D::div(PC_G * (alpha - alpha0), alpha0);
 }
-__device__ __forceinline__ double theta_rho_c(double p0, double T, double qt, double qv) {
-    return T * (1.0 - qt + PC_EPS_VI * qv) / exner_c(p0);
-}
-__device__ __forceinline__ double thetali_c(double p0, double T, double qt, double ql, double qi, double L) {
-    return T / exner_c(p0) * exp(-L * (ql / (1.0 - qt) + qi / (1.0 - qt)) / (T * PC_CPD));
-}
 
 // entropies.h:5-15
 template <class D = DivIeee> __device__ __forceinline__ double sd_c(double pd, double T) {
@@ -157,11 +151,6 @@ __device__ __forceinline__ double bvf_sa(const Table &lt, double p0, const doubl
         return D::div(PC_G, Tk) * (dTdz + gamma_w) * (1.0 + D::div(Lv * rsl, PC_RD * Tk)) - D::div(dqtdz, 1.0 - qt[1]);
     }
     return D::div(PC_G, thr[1]) * (0.5 * (thr[1] + thr[2]) - 0.5 * (thr[0] + thr[1])) * dzi;
-}
-
-// thermodynamics_dry.h:8-10
-template <class D = DivIeee> __device__ __forceinline__ double eos_dry(double pd, double s) {
-    return PC_T_TILDE * (exp(D::div(s - PC_SD_TILDE + PC_RD * log(D::div(pd, PC_P_TILDE)), PC_CPD)));
 }
 
 }  // namespace thermo
