@@ -179,3 +179,34 @@ def test_pressure_planes_stop_where_they_are_slower(lib):
         assert 0 <= form(n, 1) < 2, n
     for n in ((512, 64, 64), (512, 256, 15), (512, 32, 128), (1024, 64, 20), (1024, 16, 128), (2048, 16, 40), (4096, 8, 40)):
         assert form(n, 0) >= 2 and form(n, 1) >= 2, n
+
+
+def test_advection_chunk_search_is_short_and_exact(lib):
+    """The search for the y pass's chunks, made in every call, takes the
+    cheapest count of them all without trying them all: 100000 rows within 40 us
+    of host time (the best of 50 calls)."""
+    import time
+
+    def exhaustive(n, cols):
+        split = lambda want: (-(-n // -(-n // want)), -(-n // want))  # noqa: E731
+        want = 1
+        while cols * want < 2048 and n // (want * 2) >= 32:
+            want *= 2
+        cost, best = None, split(want)
+        while want <= n and (cost is None or n // want >= 4):
+            nch, ln = split(want)
+            c = (cols * nch + 767) // 768 * (ln + 4)
+            if cost is None or c < cost:
+                cost, best = c, (nch, ln)
+            want += 1
+        return best
+
+    for nx, ny, nz in [(64, 64, 64), (64, 64, 76), (512, 512, 256), (1024, 1024, 192), (200, 135, 75), (64, 4096, 8), (16, 1000, 8),
+                       (640, 77, 33), (24, 20, 16), (130, 2049, 5), (8, 8, 3)]:
+        assert _chunks(lib, 1, (nx, ny, nz)) == exhaustive(ny, (nx + 63) // 64 * ((nz + 3) // 4)), (nx, ny, nz)
+    best = 1.0
+    for _ in range(50):
+        t = time.perf_counter()
+        _chunks(lib, 1, (16, 100000, 8))
+        best = min(best, time.perf_counter() - t)
+    assert best < 40e-6, best
