@@ -37,6 +37,7 @@ struct pycles_pressure_plan {
     int nxh;
     int nxp;         // row stride of the spectrum: nxh rounded up to 16 (128-byte rows in FP32)
     int gx;          // kx columns per y-FFT block
+    void *mem;       // the one allocation that the arrays below lie in
     void *spec;      // [nz][ny][nxp] complex, field precision (columns nxh..nxp-1 unused)
     double *ck;      // Thomas segment carries: [nz / S][3][ny][nxp] (S levels per segment)
     double *pm;      // or, with few columns, reciprocal pivots [nz][ny nxh] and
@@ -1077,15 +1078,19 @@ extern "C" int pycles_pressure_plan_create(const pycles_dims *dims, const double
         twy[2 * m] = cos(ang);
         twy[2 * m + 1] = sin(ang);
     }
-#define ALLOC(ptr, bytes)                                   \
-    do {                                                    \
-        if (hipMalloc((void **)&(ptr), (bytes)) != hipSuccess) { \
-            pycles_set_error("pressure: hipMalloc of %zu bytes failed", (size_t)(bytes)); \
-            pycles_pressure_plan_destroy(P);                \
-            return PYCLES_ERR_HIP;                          \
-        }                                                   \
-    } while (0)
-    ALLOC(P->spec, nspec * cs);
+    // one allocation for the tables, the spectrum and the z solve's arrays (14 of
+    // them and 8 copies made a plan take 130 to 190 us) and one copy of the tables
+    struct Part {
+        void **ptr;
+        size_t off;
+    } parts[14];
+    int nparts = 0;
+    size_t total = 0;
+    auto part = [&](auto &ptr, size_t bytes) {
+        parts[nparts++] = Part{(void **)&ptr, total};
+        total += (bytes + 255) & ~(size_t)255;
+    };
+    part(P->spec, nspec * cs);
     {
         // the LDS limit is raised for every plan of the form, not to this one's size
         size_t lds;
@@ -1103,41 +1108,48 @@ extern "C" int pycles_pressure_plan_create(const pycles_dims *dims, const double
         P->planes = form == PYCLES_PRESSURE_PLANES ? 1 : form == PYCLES_PRESSURE_PLANES_STAGED ? 2 : 0;
         P->plane_lds = lds;
         if (P->planes || P->thomas_lds) {
-            ALLOC(P->pm, sizeof(double) * (size_t)g.nz * g.ny * P->nxh);
-            ALLOC(P->pc, es * (size_t)g.nz * g.ny * P->nxh);
+            part(P->pm, sizeof(double) * (size_t)g.nz * g.ny * P->nxh);
+            part(P->pc, es * (size_t)g.nz * g.ny * P->nxh);
         } else {
             const int seg = precision == PYCLES_F64 ? thomas_seg<double>() : thomas_seg<float>();
-            ALLOC(P->ck, 3 * sizeof(double) * (size_t)(g.nz / seg + 1) * g.ny * P->nxp);
+            part(P->ck, 3 * sizeof(double) * (size_t)(g.nz / seg + 1) * g.ny * P->nxp);
         }
     }
-    ALLOC(P->twx, (size_t)g.nx * cs);
-    ALLOC(P->twy, (size_t)g.ny * cs);
-    ALLOC(P->kx2, P->nxh * 8);
-    ALLOC(P->ky2, g.ny * 8);
-    ALLOC(P->rho_h, nz * 8);
-    ALLOC(P->dd, nz * 8);
-    ALLOC(P->a, nz * 8);
-    ALLOC(P->c, nz * 8);
-    ALLOC(P->mean, (size_t)g.nzg * 8);
-    ALLOC(P->partial, (size_t)g.nzg * MEAN_SPLITS * 8);
-#undef ALLOC
-    hipError_t e = hipSuccess;
-    if (precision == PYCLES_F64) {
-        e = hipMemcpy(P->twx, twx.data(), (size_t)g.nx * 16, hipMemcpyHostToDevice);
-        if (e == hipSuccess) e = hipMemcpy(P->twy, twy.data(), (size_t)g.ny * 16, hipMemcpyHostToDevice);
-    } else {
-        std::vector<float> fx(2 * g.nx), fy(2 * g.ny);
-        for (int m = 0; m < 2 * g.nx; ++m) fx[m] = (float)twx[m];
-        for (int m = 0; m < 2 * g.ny; ++m) fy[m] = (float)twy[m];
-        e = hipMemcpy(P->twx, fx.data(), (size_t)g.nx * 8, hipMemcpyHostToDevice);
-        if (e == hipSuccess) e = hipMemcpy(P->twy, fy.data(), (size_t)g.ny * 8, hipMemcpyHostToDevice);
+    part(P->mean, (size_t)g.nzg * 8);
+    part(P->partial, (size_t)g.nzg * MEAN_SPLITS * 8);
+    const size_t tab0 = total;
+    part(P->twx, (size_t)g.nx * cs);
+    part(P->twy, (size_t)g.ny * cs);
+    part(P->kx2, P->nxh * 8);
+    part(P->ky2, g.ny * 8);
+    part(P->rho_h, nz * 8);
+    part(P->dd, nz * 8);
+    part(P->a, nz * 8);
+    part(P->c, nz * 8);
+    std::vector<unsigned char> tables(total - tab0);
+    if (hipMalloc(&P->mem, total) != hipSuccess) {
+        (void)hipGetLastError();
+        pycles_set_error("pressure: hipMalloc of %zu bytes failed", total);
+        pycles_pressure_plan_destroy(P);
+        return PYCLES_ERR_HIP;
     }
-    if (e == hipSuccess) e = hipMemcpy(P->kx2, kx2.data(), P->nxh * 8, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(P->ky2, ky2.data(), g.ny * 8, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(P->rho_h, rh.data(), nz * 8, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(P->dd, dd.data(), nz * 8, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(P->a, a.data(), nz * 8, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(P->c, c.data(), nz * 8, hipMemcpyHostToDevice);
+    for (int q = 0; q < nparts; ++q) *parts[q].ptr = (char *)P->mem + parts[q].off;
+    auto put = [&](const void *dev, const double *v, int n, bool field) {
+        unsigned char *h = tables.data() + ((const char *)dev - (const char *)P->mem - tab0);
+        if (field && precision == PYCLES_F32)
+            for (int m = 0; m < n; ++m) ((float *)h)[m] = (float)v[m];
+        else
+            memcpy(h, v, n * sizeof(double));
+    };
+    put(P->twx, twx.data(), 2 * g.nx, true);
+    put(P->twy, twy.data(), 2 * g.ny, true);
+    put(P->kx2, kx2.data(), P->nxh, false);
+    put(P->ky2, ky2.data(), g.ny, false);
+    put(P->rho_h, rh.data(), nz, false);
+    put(P->dd, dd.data(), nz, false);
+    put(P->a, a.data(), nz, false);
+    put(P->c, c.data(), nz, false);
+    hipError_t e = hipMemcpy((char *)P->mem + tab0, tables.data(), tables.size(), hipMemcpyHostToDevice);
     if (e != hipSuccess) {
         pycles_set_error("pressure: table upload failed: %s", hipGetErrorString(e));
         pycles_pressure_plan_destroy(P);
@@ -1168,10 +1180,7 @@ extern "C" int pycles_pressure_plan_create(const pycles_dims *dims, const double
 
 extern "C" void pycles_pressure_plan_destroy(pycles_pressure_plan *P) {
     if (!P) return;
-    void *ptrs[] = {P->spec, P->ck, P->pm, P->pc, P->twx, P->twy, P->kx2, P->ky2, P->rho_h,
-                    P->dd, P->a, P->c, P->mean, P->partial};
-    for (void *p : ptrs)
-        if (p) (void)hipFree(p);
+    if (P->mem) (void)hipFree(P->mem);
     delete P;
 }
 
