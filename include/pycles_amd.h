@@ -191,7 +191,7 @@ int pycles_forcing_bomex(const pycles_dims *dims, const pycles_ref *ref, const d
                          double coriolis, double u0, double v0, int precision, void *stream);
 /* Replaces Rayleigh.update (Damping.pyx:95-133) for nv (<= 8) fields:
  * tend -= (phi - mean_k(phi)) gamma[v][k] over the interior, means = [nv][nzg]
- * the level means of the stored fields (pycles_level_mean), gamma[v] the
+ * the level means of the stored fields (pycles_level_means), gamma[v] the
  * profile of field v (the reference uses the half-level profile for w and
  * the full-level one for the others). */
 int pycles_rayleigh_damping(const pycles_dims *dims, int nv, const void *const *fields, void *const *tend,
@@ -298,7 +298,9 @@ int pycles_pressure_form(const pycles_dims *dims, int precision);
  * pressure z boundary fill, u -= grad p, boundary fill of u, v, w.
  * p (dynamic pressure) and div (may be NULL) use the field precision.
  * If cfl_out is non-NULL the CFL maximum of the corrected velocities
- * (as pycles_cfl_max with dt) is written there too. */
+ * (as pycles_cfl_max with dt) is written there too: one FP64 value in device
+ * memory, as out of pycles_cfl_max (the blocks' maxima meet there by atomics,
+ * from zero, which an earlier kernel of the call stores). */
 int pycles_pressure_update(pycles_pressure_plan *plan, const pycles_ref *ref, void *u, void *v,
                            void *w, void *p, void *div, double dt, double *cfl_out, void *stream);
 /* second_order_divergence of the current velocities (interior, field precision). */

@@ -8,7 +8,7 @@ wind, radiative cooling, drying, subsidence; the damping coefficients) are
 built once on the host with the reference's expressions, copied to HBM, and
 every per-cell update runs in ``pycles_surface_bomex``,
 ``pycles_forcing_bomex`` and ``pycles_rayleigh_damping``.  Horizontal means
-come from ``pycles_level_mean``.  Other cases' surface and forcing schemes
+come from ``pycles_level_means``.  Other cases' surface and forcing schemes
 are not on the device path.
 """
 from __future__ import annotations

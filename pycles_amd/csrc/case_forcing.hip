@@ -11,7 +11,7 @@
 // All three add to the tendencies after the advection, in the reference's
 // order within each variable.  The horizontal means they need (u and v for
 // the geostrophic term, every variable for the damping, T at the first level
-// for the surface diagnostics) come from pycles_level_mean beforehand.
+// for the surface diagnostics) come from pycles_level_means beforehand.
 #include "common.h"
 #include "thermo_funcs.h"
 

@@ -369,10 +369,12 @@ template <typename T> struct Interp<7, T> {
     }
     // weno() of a stencil whose centre value q[3] is zero (offsets from the
     // centre), for the FP32 form: without the centre's terms, 79 operations and
-    // 5 reciprocals against 108 and 5, and the same bits: where a centre's term
-    // was the partner of a product in a multiply-add, mul_rn leaves that product
-    // rounded by itself.  200 x 135 x 75 WENO7 tendencies 185 -> 159 us, with the
-    // profile rows of the z pass (advection_impl.h).
+    // 5 reciprocals against 108 and 5, each rounded as in weno(): where a centre's
+    // term was the partner of a product in a multiply-add, mul_rn leaves that
+    // product rounded by itself.  The tendencies of the x and y passes and the
+    // momentum's of the z pass keep their bits on 200 x 136 x 75 (the scalars' of
+    // the z pass moved with the profile rows, advection_impl.h).  200 x 135 x 75
+    // WENO7 tendencies 185 -> 159 us, with those rows.
     static __device__ __forceinline__ T weno_c0(const T *q) {
         const T m3 = q[0], m2 = q[1], m1 = q[2], p1 = q[4], p2 = q[5], p3 = q[6];
         const T s0 = T(-1.0 / 4.0) * m3 + T(13.0 / 12.0) * m2 + T(-23.0 / 12.0) * m1;
@@ -442,9 +444,9 @@ template <typename T> struct Interp<9, T> {
         return w0 * s0 + w1 * s1 + w2 * s2 + w3 * s3 + w4 * s4;
     }
     // weno() of a stencil whose centre value q[4] is zero, without its terms
-    // (see order 7): 129 operations and 6 reciprocals against 174 and 6, the same
-    // bits.  1024 x 1024 x 192 WENO9/5 tendencies 12.3 -> 11.3 ms, with the profile
-    // rows.
+    // (see order 7): 129 operations and 6 reciprocals against 174 and 6, each
+    // rounded as in weno().  1024 x 1024 x 192 WENO9/5 tendencies 12.3 -> 11.3 ms,
+    // with the profile rows.
     static __device__ __forceinline__ T weno_c0(const T *q) {
         const T m4 = q[0], m3 = q[1], m2 = q[2], m1 = q[3], p1 = q[5], p2 = q[6], p3 = q[7], p4 = q[8];
         const T s0 = T(1.0 / 5.0) * m4 + T(-21.0 / 20.0) * m3 + T(137.0 / 60.0) * m2 + T(-163.0 / 60.0) * m1;
